@@ -286,17 +286,11 @@ struct HitEval {
     float ghat;
     float u, v, t;   // ray-branch coordinates (t = centre depth on the screen branch)
     float inv_d;     // 1 / D (ray branch)
+    float uv2;       // u^2 + v^2
+    float raw;       // o * ghat
     bool ray;
     bool clamped;    // o * ghat > 0.995
 };
-
-// Exponent threshold below which a record cannot reach alpha >= 1/255:
-// o * exp(e) >= 1/255 needs e >= -ln(255 o); the 1e-3 slack (a 0.1 % factor)
-// dwarfs the error of __expf, so skipping e < lthr never drops a
-// contribution the exact test would keep.
-__device__ __forceinline__ float record_lthr(float opacity) {
-    return opacity * 255.0f > 1.0f ? -(logf(opacity * 255.0f) + 1e-3f) : 1.0f;  // 1 > any e: never
-}
 
 // Conservative footprint of a record: the pixels at which it can reach
 // alpha >= 1/255 lie in the screen low-pass disk dx^2 + dy^2 <= L around
@@ -445,6 +439,68 @@ __device__ __forceinline__ uint32_t block_mask(const Record& r, uint32_t x0, uin
     return m;
 }
 
+// Footprint against the 4x4 sub-blocks of a tile, one row of sub-blocks at a
+// time: the ellipse's and the disk's x extents over the row's y range give a
+// column interval, cut by the box. In offsets from the centre the ellipse is
+// x = -k y -+ sqrt(i00 - q y^2), k = h01 / h00, q = det / h00^2; over a y
+// interval its right edge is concave with its maximum at y = -ys (the
+// ellipse's own extreme) and its left edge convex with its minimum at ys, so
+// each is evaluated at that y clamped to the interval. The same 1 px of
+// margin as footprint_hits, and the hull of the two extents: never fewer
+// sub-blocks than the record reaches.
+struct SubTest {
+    float4 box;
+    float px, py, rd2;             // screen disk
+    float ex, ey, k, q, i00, ys;   // ellipse; i00 = 0: unbounded (the box decides)
+};
+__device__ __forceinline__ SubTest sub_test(float4 box, float4 e0, float4 e1, float px, float py) {
+    SubTest t;
+    t.box = box;
+    t.px = px;
+    t.py = py;
+    t.rd2 = e1.w * e1.w;
+    t.ex = e0.x;
+    t.ey = e0.y;
+    const float det = fmaf(e0.z, e1.x, -e0.w * e0.w);
+    t.i00 = e1.y;
+    t.k = e0.w * e1.y;
+    t.q = det * e1.y * e1.y;
+    // ys = h01 / h11 * sqrt(h11 / det).
+    t.ys = e0.w * e1.z * __builtin_amdgcn_sqrtf(e1.x * __builtin_amdgcn_rcpf(det));
+    return t;
+}
+// Bit c: the record's footprint can reach the sub-block of pixel centres
+// [x0 + 4 c + 0.5, + 3] x [y0 + 0.5, + 3].
+__device__ __forceinline__ uint32_t sub_row_mask(const SubTest& t, float x0, float y0) {
+    const float ylo = y0 + 0.5f, yhi = y0 + 3.5f;
+    float xl, xr;
+    if (t.i00 == 0.0f) {
+        xl = -kFar;
+        xr = kFar;
+    } else {
+        const float da = ylo - 1.0f - t.ey, db = yhi + 1.0f - t.ey;
+        const float yr = fminf(fmaxf(-t.ys, da), db), yl = fminf(fmaxf(t.ys, da), db);
+        const float dr = fmaf(-t.q * yr, yr, t.i00), dl = fmaf(-t.q * yl, yl, t.i00);
+        // The strip meets the ellipse in both or in neither (rounding aside).
+        const float slack = -1e-3f * t.i00;
+        const bool hit = dr >= slack || dl >= slack;
+        xr = hit ? t.ex - t.k * yr + __builtin_amdgcn_sqrtf(fmaxf(dr, 0.0f)) : -kFar;
+        xl = hit ? t.ex - t.k * yl - __builtin_amdgcn_sqrtf(fmaxf(dl, 0.0f)) : kFar;
+        const float dy = fminf(fmaxf(t.py, ylo - 1.0f), yhi + 1.0f) - t.py;
+        const float h2 = fmaf(-dy, dy, t.rd2);
+        const float hx = __builtin_amdgcn_sqrtf(fmaxf(h2, 0.0f));
+        xr = h2 >= 0.0f ? fmaxf(xr, t.px + hx) : xr;
+        xl = h2 >= 0.0f ? fminf(xl, t.px - hx) : xl;
+    }
+    // Columns [lo, hi]: x0 + 4 c + 3.5 (+ 1) >= left edge, x0 + 4 c + 0.5 (- 1) <= right edge.
+    const float lo = fmaxf(xl - 4.5f, t.box.x - 3.5f) - x0, hi = fminf(xr + 0.5f, t.box.z - 0.5f) - x0;
+    const int cl = (int)ceilf(fminf(fmaxf(lo * 0.25f, 0.0f), 4.0f));
+    const int ch = (int)floorf(fminf(fmaxf(hi * 0.25f, -1.0f), 3.0f));
+    const uint32_t m = ((1u << (ch + 1)) - 1u) & ~((1u << cl) - 1u);
+    const bool rows = t.box.w >= ylo && t.box.y <= yhi && ch >= 0;
+    return rows ? m : 0u;
+}
+
 // Cuts a footprint box (pixel centres) to the pixels of the kTile rect
 // (x0, y0, x1, y1, inclusive): pixels outside the rect are not reached in the
 // forward model (forward.rs:104-123), whatever the footprint.
@@ -478,8 +534,7 @@ __device__ __forceinline__ float rcp_refined(float x) {
     return fmaf(r0, fmaf(-x, r0, 1.0f), r0);
 }
 
-__device__ __forceinline__ HitEval eval_hit(const Record& r, float sx, float sy, float pxc, float pyc,
-                                            float lthr = -INFINITY) {
+__device__ __forceinline__ HitEval eval_hit(const Record& r, float sx, float sy, float pxc, float pyc) {
     HitEval h;
     // D = M.s, Nu = A.s, Nv = B.s with s = (sx, sy, 1): two FMAs each.
     const float D = fmaf(r.m_nt.x, sx, fmaf(r.m_nt.y, sy, r.m_nt.z));
@@ -494,20 +549,18 @@ __device__ __forceinline__ HitEval eval_hit(const Record& r, float sx, float sy,
     h.v = Nv * inv;
     h.t = r.m_nt.w * inv;
     h.inv_d = inv;
-    const float e_ray = h.t > kNearDepth ? -(h.u * h.u + h.v * h.v) * 0.5f : -INFINITY;
+    // Explicit fmaf: every kernel that evaluates a hit rounds it alike.
+    h.uv2 = fmaf(h.u, h.u, h.v * h.v);
+    const float e_ray = h.t > kNearDepth ? -h.uv2 * 0.5f : -INFINITY;
     const float dx = pxc - r.a_px.w, dy = pyc - r.b_py.w;
-    const float e_scr = -(dx * dx + dy * dy);   // 2 sigma^2 = 1 (LOWPASS_SIGMA2 = 0.5)
+    const float e_scr = -fmaf(dx, dx, dy * dy);   // 2 sigma^2 = 1 (LOWPASS_SIGMA2 = 0.5)
     h.ray = e_ray >= e_scr;
     const float e = h.ray ? e_ray : e_scr;
     if (!h.ray) h.t = r.nrm_dep.w;
-    // e < lthr cannot reach 1/255 (see record_lthr): ghat = 0, hence alpha
-    // = 0 and no clamp. A select, not a branch: exp runs on every lane (e is
-    // finite, the screen term bounds it below), and no lane's state forks.
-    const float g = __expf(e);
-    h.ghat = e < lthr ? 0.0f : g;
-    const float raw = r.col_op.w * h.ghat;
-    h.clamped = raw > kAlphaClamp;
-    float a = fminf(raw, kAlphaClamp);
+    h.ghat = __expf(e);
+    h.raw = r.col_op.w * h.ghat;
+    h.clamped = h.raw > kAlphaClamp;
+    float a = fminf(h.raw, kAlphaClamp);
     h.alpha = a < kAlphaSkip ? 0.0f : a;
     return h;
 }
@@ -666,12 +719,42 @@ struct BwdIn {
     const float4* out_aux;     // T_final, sum w t
     const uint32_t* ncontrib;
 };
+// Long tile lists of the backward, split over depth (16-px tiles, with a tile
+// queue): raster_state_kernel walks a long list back to front, keeping only
+// each pixel's T and suffix sums, and stores them at the segment boundaries;
+// the gradient pass then takes every segment as a unit of its own. A tile's
+// walk is sequential in depth, so without this the longest list is the
+// launch's critical path. state == nullptr: off.
+constexpr uint32_t kSegmentPool = 12288;   // segments of one pass
+constexpr uint32_t kSegmentTarget = 6144;  // a segment holds at least 1 / this of the entries
+constexpr uint32_t kSegmentMin = 32;       // and at least this many records
+constexpr uint32_t kSegmentPixels = 256;
+constexpr uint32_t kSegmentLast = 1u << 31;
+struct BwdSegments {
+    uint32_t* ctl = nullptr;     // [0] segments in use, [1] records per segment
+    uint2* table = nullptr;      // per segment: tile, index | kSegmentLast (tile ~0: none)
+    uint32_t* split = nullptr;   // per tile: 1 = walked by segments
+    float4* state = nullptr;     // [1, with aux 3][pool][kSegmentPixels]
+    uint32_t pool = 0;
+};
+// Split tiles' lists are longer than a segment of at least E / kSegmentTarget
+// (E = entries) and at least kSegmentMin records, so a tile has at most 2 len
+// / L of them and all have at most 2 E / L.
+constexpr uint32_t segment_pool(uint32_t max_entries) {
+    const uint64_t most = 2ull * max_entries / kSegmentMin + 16;
+    return (uint32_t)(most < kSegmentPool + 16 ? most : kSegmentPool + 16);
+}
+// Clears the gradient accumulator (floats a multiple of 4) and readies a
+// backward pass: the queue's cursors (optional), the split flags of
+// split_tiles tiles and the segment length for *entries entries.
+hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
+                              uint32_t split_tiles, const uint32_t* entries);
 hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const CamParams* cams_host,
                              uint32_t n_views, uint32_t total_tiles, const uint32_t* ranges,
                              const uint32_t* payloads, const Record* recs, BwdIn in,
                              float* grad_coef, bool aux, bool cull = true,
                              TileQueue queue = {nullptr, nullptr, 0}, RasterShape shape = {},
-                             uint32_t tile_begin = 0);
+                             uint32_t tile_begin = 0, BwdSegments sg = {});
 
 // geom_bwd.hip
 struct ParamGrads {

@@ -17,12 +17,16 @@
 //     gradient with hardware global FP32 atomics (no CAS loops). A 32x32
 //     tile is eight waves, each owning an 8-wide, 16-tall column of two
 //     blocks (two pixels per lane), whose per-record reductions meet in LDS
-//     slots (ds_add_f32) flushed once per batch; an 8x8 tile is one wave with
+//     slots (ds_add_f32) flushed once per batch (the two waves of the depth /
+//     normal variant each have a copy of them); an 8x8 tile is one wave with
 //     one pixel per lane (raster_bwd_kernel). Records are staged BATCH at a
 //     time into order-preserving lists that carry the blocks each reaches;
 //   * each wave reduces its lanes' 16 values with a transposed butterfly (17
 //     lane exchanges instead of 96, on permlane swaps and DPP rather than LDS
-//     permutes).
+//     permutes);
+//   * lists longer than a segment are split over depth: a state pass
+//     (raster_state_kernel) leaves each pixel's walk state at the segment
+//     boundaries, and the gradient pass takes segments as units.
 // AUX = true (16-px tiles, raster_bwd_kernel) adds the depth / normal image
 // losses and the in-walk depth distortion loss (backward.rs:126-153).
 
@@ -147,6 +151,104 @@ __device__ __forceinline__ void load_pixel(PixState& p, const CamParams& cam, in
     p.last = has_loss ? last : 0u;
 }
 
+// The walk state's own arithmetic is written with explicit fmaf: the state
+// pass (raster_state_kernel) has to reach the gradient pass's values bit for
+// bit, which contraction left to the compiler would not promise.
+// d(distortion)/dw of a hit and, in dt_dist, its derivative with respect to
+// the hit's depth (backward.rs:126-153).
+__device__ __forceinline__ float distortion_coef(const PixState& p, float w, float t_hit, float lambda,
+                                                 float& dt_dist) {
+    if (lambda == 0.0f) return 0.0f;
+    const float a_pre = p.w_total - p.suf_w - w;
+    const float b_pre = fmaf(-w, t_hit, p.wt_total - p.suf_d);
+    dt_dist = lambda * 2.0f * w * (a_pre - p.suf_w);
+    return lambda * fmaf(2.0f, fmaf(t_hit, a_pre, -b_pre), 2.0f * fmaf(-t_hit, p.suf_w, p.suf_d));
+}
+__device__ __forceinline__ void step_aux_sums(PixState& p, const Record& r, float w, float t_hit, float coef) {
+    p.suf_d = fmaf(t_hit, w, p.suf_d);
+    p.suf_nx = fmaf(r.nrm_dep.x, w, p.suf_nx);
+    p.suf_ny = fmaf(r.nrm_dep.y, w, p.suf_ny);
+    p.suf_nz = fmaf(r.nrm_dep.z, w, p.suf_nz);
+    p.suf_w += w;
+    p.suf_cw = fmaf(coef, w, p.suf_cw);
+}
+// One record's step of the walk without its gradient terms: what add_hit
+// does to T and the suffix sums.
+template <bool AUX>
+__device__ __forceinline__ void step_state(PixState& p, const Record& r, const HitEval& h, bool act, float lambda) {
+    const float alpha = act ? h.alpha : 0.0f;
+    const float t_before = p.T * rcp_refined(1.0f - alpha);
+    const float w = t_before * alpha;
+    p.suf_r = fmaf(r.col_op.x, w, p.suf_r);
+    p.suf_g = fmaf(r.col_op.y, w, p.suf_g);
+    p.suf_b = fmaf(r.col_op.z, w, p.suf_b);
+    if (AUX) {
+        float dt_dist = 0.0f;
+        const float coef = distortion_coef(p, w, h.t, lambda, dt_dist);
+        step_aux_sums(p, r, w, h.t, coef);
+    }
+    p.T = t_before;
+}
+
+// Walk states at segment boundaries (BwdSegments::state): pixel k of the
+// tile (8x8 block k >> 6, row-major within it) of segment `at`.
+template <bool AUX>
+__device__ __forceinline__ void store_state(const BwdSegments& sg, uint32_t at, uint32_t k, const PixState& p) {
+    float4* dst = sg.state + (size_t)at * kSegmentPixels + k;
+    const size_t plane = (size_t)sg.pool * kSegmentPixels;
+    dst[0] = make_float4(p.T, p.suf_r, p.suf_g, p.suf_b);
+    if (AUX) {
+        dst[plane] = make_float4(p.suf_d, p.suf_nx, p.suf_ny, p.suf_nz);
+        dst[2 * plane] = make_float4(p.suf_w, p.suf_cw, 0.0f, 0.0f);
+    }
+}
+template <bool AUX>
+__device__ __forceinline__ void load_state(const BwdSegments& sg, uint32_t at, uint32_t k, PixState& p) {
+    const float4* src = sg.state + (size_t)at * kSegmentPixels + k;
+    const size_t plane = (size_t)sg.pool * kSegmentPixels;
+    const float4 a = src[0];
+    p.T = a.x;
+    p.suf_r = a.y;
+    p.suf_g = a.z;
+    p.suf_b = a.w;
+    if (AUX) {
+        const float4 b = src[plane], c = src[2 * plane];
+        p.suf_d = b.x;
+        p.suf_nx = b.y;
+        p.suf_ny = b.z;
+        p.suf_nz = b.w;
+        p.suf_w = c.x;
+        p.suf_cw = c.y;
+    }
+}
+
+// One unit of the gradient pass: a tile, and either its whole list (seg ==
+// kWholeTile) or one segment of it.
+constexpr uint32_t kWholeTile = ~0u;
+struct BwdItem {
+    uint32_t tile, seg, at;  // at: the segment's slot (its boundary state)
+    bool last;               // the tile's last segment: starts from the forward's end
+};
+// Position pos of the pass: the segments first (the largest units), then the
+// tiles in the queue's order, of which the split ones are done already.
+// False: nothing to do at this position.
+__device__ __forceinline__ bool bwd_item(const BwdSegments& sg, uint32_t nseg, uint32_t pos, const TileQueue& queue,
+                                         uint32_t tile_begin, BwdItem& it) {
+    it.seg = kWholeTile;
+    it.at = 0;
+    it.last = true;
+    if (pos < nseg) {
+        const uint2 e = sg.table[pos];
+        it.tile = e.x;
+        it.seg = e.y & ~kSegmentLast;
+        it.last = (e.y & kSegmentLast) != 0u;
+        it.at = pos;
+        return e.x != ~0u;
+    }
+    it.tile = queue.order != nullptr ? queue.order[pos - nseg] : tile_begin + (pos - nseg);
+    return sg.state == nullptr || sg.split[it.tile] == 0u;
+}
+
 template <bool AUX, bool ACC>
 __device__ __forceinline__ void put(float& dst, float v) {
     if constexpr (ACC) dst += v;
@@ -173,17 +275,12 @@ __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitE
     float dl_dt = 0.0f;
     float dl_dalpha = (p.dlr * r.col_op.x + p.dlg * r.col_op.y + p.dlb * r.col_op.z) * t_before -
                       (p.dlr * p.suf_r + p.dlg * p.suf_g + p.dlb * p.suf_b) * inv_one_m;
-    p.suf_r += r.col_op.x * w;
-    p.suf_g += r.col_op.y * w;
-    p.suf_b += r.col_op.z * w;
+    p.suf_r = fmaf(r.col_op.x, w, p.suf_r);
+    p.suf_g = fmaf(r.col_op.y, w, p.suf_g);
+    p.suf_b = fmaf(r.col_op.z, w, p.suf_b);
     if (AUX) {
-        float dt_dist = 0.0f, coef = 0.0f;
-        if (lambda != 0.0f) {
-            const float a_pre = p.w_total - p.suf_w - w;
-            const float b_pre = p.wt_total - p.suf_d - w * t_hit;
-            dt_dist = lambda * 2.0f * w * (a_pre - p.suf_w);
-            coef = lambda * (2.0f * (t_hit * a_pre - b_pre) + 2.0f * (p.suf_d - t_hit * p.suf_w));
-        }
+        float dt_dist = 0.0f;
+        const float coef = distortion_coef(p, w, t_hit, lambda, dt_dist);
         put<AUX, ACC>(g2[kGNrm - 16 + 0], p.dnx * w);
         put<AUX, ACC>(g2[kGNrm - 16 + 1], p.dny * w);
         put<AUX, ACC>(g2[kGNrm - 16 + 2], p.dnz * w);
@@ -192,12 +289,7 @@ __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitE
                      (p.dnx * r.nrm_dep.x + p.dny * r.nrm_dep.y + p.dnz * r.nrm_dep.z) * t_before -
                      (p.dnx * p.suf_nx + p.dny * p.suf_ny + p.dnz * p.suf_nz) * inv_one_m +
                      coef * t_before - p.suf_cw * inv_one_m;
-        p.suf_d += t_hit * w;
-        p.suf_nx += r.nrm_dep.x * w;
-        p.suf_ny += r.nrm_dep.y * w;
-        p.suf_nz += r.nrm_dep.z * w;
-        p.suf_w += w;
-        p.suf_cw += coef * w;
+        step_aux_sums(p, r, w, t_hit, coef);
     }
     p.T = t_before;
     // Geometry terms exist only for contributing, unclamped hits, and the
@@ -241,7 +333,8 @@ template <bool AUX, int TW, int BATCH>
 __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in,
-    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin) {
+    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
+    BwdSegments sg) {
     constexpr int NS = grad_stride(AUX);     // slots per record (LDS and grad_coef)
     constexpr bool TWO = TW >= 16;           // two pixels per lane (an 8x16 column per wave)
     constexpr int NC = TW / 8;               // 8x8 blocks per tile row
@@ -252,11 +345,14 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     constexpr int MB = 10;                   // list entry: slot | top << MB | bottom << (MB + 1)
     static_assert(BATCH % 64 == 0 && BATCH <= (1 << MB), "batch of whole waves");
     __shared__ float4 s_m[BATCH], s_a[BATCH], s_b[BATCH], s_c[BATCH], s_n[AUX ? BATCH : 1];
-    __shared__ float s_lthr[BATCH];
     __shared__ uint32_t s_pay[BATCH];        // the batch's surfel ids, for the flush
     __shared__ uint16_t s_list[NW][BATCH];
     __shared__ uint32_t s_qcnt[SW][NW];      // [staging wave][list wave]
-    __shared__ float s_grad[BATCH * NS];
+    // One or two waves: a copy of the slots per wave, written (a wave meets a
+    // record once per batch) and summed at the flush; LDS float atomics run at
+    // one lane per ~3 cycles. Eight waves (32-px tiles) share one copy.
+    constexpr int NG = NW <= 2 ? NW : 1;
+    __shared__ float s_grad[NG][BATCH * NS];
     __shared__ uint32_t s_view, s_maxlast, s_next;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -264,9 +360,13 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     // Wave w owns block column c = w % NC, rows 16 (w / NC) .. + 15: blocks
     // top = (c, 2 (w / NC)) and bottom = (c, 2 (w / NC) + 1).
     const int col = wave % NC, hrow = wave / NC;
+    const uint32_t nseg = sg.state != nullptr ? min(sg.ctl[0], sg.pool) : 0u;
+    const uint32_t items = total_tiles + nseg;
+    // Room for every item: each workgroup takes one, without a claim.
+    const bool claim = queue.cursor != nullptr && items > gridDim.x;
     for (uint32_t iter = 0;; ++iter) {
         uint32_t pos;
-        if (queue.cursor != nullptr) {
+        if (claim) {
             if (tid == 0) {
                 const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
                 s_next = atomicAdd(queue.cursor + x, 1u) * q + x;
@@ -275,10 +375,12 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
             pos = s_next;
             __syncthreads();  // every thread has pos before s_next is rewritten
         } else {
-            pos = iter == 0 ? xcd_swizzle(blockIdx.x, gridDim.x) : total_tiles;
+            pos = iter > 0 ? items : queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
         }
-        if (pos >= total_tiles) break;
-        const uint32_t gtile = queue.order != nullptr ? queue.order[pos] : tile_begin + pos;
+        if (pos >= items) break;
+        BwdItem it;
+        if (!bwd_item(sg, nseg, pos, queue, tile_begin, it)) continue;
+        const uint32_t gtile = it.tile;
         const uint32_t start = ranges[2 * (size_t)gtile], end = ranges[2 * (size_t)gtile + 1];
         if (end <= start) continue;
         if (tid == 0) {
@@ -302,11 +404,25 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
         __syncthreads();
         const uint32_t maxlast = s_maxlast;
         if (maxlast == 0) continue;
+        // The list positions [k0, k1) of this item.
+        uint32_t k0 = 0, k1 = maxlast;
+        if (it.seg != kWholeTile) {
+            k0 = it.seg * sg.ctl[1];
+            if (!it.last) {
+                k1 = k0 + sg.ctl[1];
+                if constexpr (TW == 16) {
+                    const uint32_t k = (uint32_t)(col + 2 * (2 * hrow)) * 64u + (uint32_t)lane;
+                    load_state<AUX>(sg, it.at, k, pa);
+                    load_state<AUX>(sg, it.at, k + 128u, pb);
+                }
+            }
+        }
 
-        const int nbatch = (int)((maxlast + BATCH - 1) / BATCH);
+        const int nbatch = (int)((k1 - k0 + BATCH - 1) / BATCH);
         for (int b = nbatch - 1; b >= 0; --b) {
-            const uint32_t base = start + (uint32_t)b * BATCH;
-            const uint32_t cnt = min(min((uint32_t)BATCH, end - base), maxlast - (uint32_t)b * BATCH);
+            const uint32_t first = k0 + (uint32_t)b * BATCH;
+            const uint32_t base = start + first;
+            const uint32_t cnt = min((uint32_t)BATCH, k1 - first);
             uint32_t memb[SPT][NW], qpos[SPT][NW];
 #pragma unroll
             for (int m = 0; m < SPT; ++m) {
@@ -322,7 +438,6 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                     s_b[slot] = r.b_py;
                     s_c[slot] = r.col_op;
                     if (AUX) s_n[slot] = r.nrm_dep;
-                    s_lthr[slot] = record_lthr(r.col_op.w);
                     qmask = cull ? block_mask<TW>(r, x0, y0) : ~0u;
                 }
                 // Order-preserving per-wave lists: wave w takes the records
@@ -339,7 +454,10 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                     if (lane == 0) s_qcnt[sw][w] = (uint32_t)__popcll(bal);
                 }
             }
-            for (int k = tid; k < (int)cnt * NS; k += NT) s_grad[k] = 0.0f;
+            for (int k = tid; k < (int)cnt * NS; k += NT) {
+#pragma unroll
+                for (int c = 0; c < NG; ++c) s_grad[c][k] = 0.0f;
+            }
             __syncthreads();
 #pragma unroll
             for (int m = 0; m < SPT; ++m) {
@@ -366,7 +484,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 const uint32_t e = __builtin_amdgcn_readfirstlane((uint32_t)s_list[wave][kk]);
                 const uint32_t j = e & ((1u << MB) - 1u);
                 const bool top = (e >> MB) & 1u, bot = TWO && ((e >> (MB + 1)) & 1u);
-                const uint32_t rel = (uint32_t)b * BATCH + j;
+                const uint32_t rel = first + j;
                 // A block is walked only while some pixel of it is at or before
                 // its last contributor (a pixel past it changes nothing).
                 const bool need_a = top && __any(rel < pa.last);
@@ -378,18 +496,17 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 r.b_py = s_b[j];
                 r.col_op = s_c[j];
                 r.nrm_dep = AUX ? s_n[AUX ? j : 0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                const float lthr = s_lthr[j];
                 // Evaluate first; the gradient terms and the reduction run only
                 // for blocks with a contributing lane (for the others the walk
                 // state would not change).
                 HitEval ha, hb;
                 bool act_a = false, act_b = false;
                 if (need_a) {
-                    ha = eval_hit(r, pa.sx, pa.sy, pa.pxc, pa.pyc, lthr);
+                    ha = eval_hit(r, pa.sx, pa.sy, pa.pxc, pa.pyc);
                     act_a = rel < pa.last && ha.alpha > 0.0f;
                 }
                 if (need_b) {
-                    hb = eval_hit(r, pb.sx, pb.sy, pb.pxc, pb.pyc, lthr);
+                    hb = eval_hit(r, pb.sx, pb.sy, pb.pxc, pb.pyc);
                     act_b = rel < pb.last && hb.alpha > 0.0f;
                 }
                 const bool go_a = need_a && __any(act_a);
@@ -410,16 +527,20 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 }
                 const float red = wave_reduce_transpose<16>(g, lane);
                 if ((lane & 3) == 0) {
-                    if (red != 0.0f) atomicAdd(&s_grad[j * NS + (lane >> 2)], red);
+                    float* const dst = &s_grad[NG > 1 ? wave : 0][j * NS + (lane >> 2)];
+                    if constexpr (NG == NW) *dst = red;
+                    else if (red != 0.0f) atomicAdd(dst, red);
                 }
                 if (AUX) {
+                    static_assert(!AUX || NG == NW, "a copy of the slots per wave");
                     const float red2 = wave_reduce_transpose<4>(g2, lane);
-                    if ((lane & 15) == 0 && red2 != 0.0f) atomicAdd(&s_grad[j * NS + 16 + (lane >> 4)], red2);
+                    if ((lane & 15) == 0) s_grad[NG > 1 ? wave : 0][j * NS + 16 + (lane >> 4)] = red2;
                 }
             }
             __syncthreads();
             for (int k = tid; k < (int)cnt * NS; k += NT) {
-                const float v = s_grad[k];
+                float v = s_grad[0][k];
+                if constexpr (NG == 2) v += s_grad[1][k];
                 if (v != 0.0f) {
                     const int e = k / NS, slot = k - e * NS;
                     // A colour channel clamped at 0 in the forward passes no
@@ -449,21 +570,25 @@ template <int BATCH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void raster_bwd_wave_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in,
-    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin) {
+    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
+    BwdSegments sg) {
     constexpr int NS = grad_stride(false);
     constexpr int SPT = BATCH / 64;          // staging rounds per batch
     constexpr int MB = 10;                   // list entry: slot | block mask << MB
     static_assert(BATCH % 64 == 0 && BATCH <= (1 << MB), "batch of whole waves");
     __shared__ float4 s_m[BATCH], s_a[BATCH], s_b[BATCH], s_c[BATCH];
-    __shared__ float s_lthr[BATCH];
     __shared__ uint32_t s_pay[BATCH];
     __shared__ uint16_t s_list[BATCH];
 
     const int lane = threadIdx.x;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t nseg = sg.state != nullptr ? min(sg.ctl[0], sg.pool) : 0u;
+    const uint32_t items = total_tiles + nseg;
+    // Room for every item: each wave takes one, without a claim.
+    const bool claims = queue.cursor != nullptr && items > gridDim.x;
     for (uint32_t iter = 0;; ++iter) {
         uint32_t pos;
-        if (queue.cursor != nullptr) {
+        if (claims) {
             uint32_t claim = 0;
             if (lane == 0) {
                 const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
@@ -471,10 +596,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
             }
             pos = __builtin_amdgcn_readfirstlane(claim);
         } else {
-            pos = iter == 0 ? xcd_swizzle(blockIdx.x, gridDim.x) : total_tiles;
+            pos = iter > 0 ? items : queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
         }
-        if (pos >= total_tiles) break;
-        const uint32_t gtile = queue.order != nullptr ? queue.order[pos] : tile_begin + pos;
+        if (pos >= items) break;
+        BwdItem it;
+        if (!bwd_item(sg, nseg, pos, queue, tile_begin, it)) continue;
+        const uint32_t gtile = it.tile;
         const uint32_t start = ranges[2 * (size_t)gtile], end = ranges[2 * (size_t)gtile + 1];
         if (end <= start) continue;
         const uint32_t v = view_of_tile(cams, n_views, gtile);
@@ -493,11 +620,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
         for (int o = 32; o >= 1; o >>= 1) mylast = max(mylast, (uint32_t)__shfl_xor((int)mylast, o));
         const uint32_t maxlast = __builtin_amdgcn_readfirstlane(mylast);
         if (maxlast == 0) continue;
+        // The list positions [k0, k1) of this item.
+        uint32_t k0 = 0, k1 = maxlast;
+        if (it.seg != kWholeTile) {
+            k0 = it.seg * sg.ctl[1];
+            if (!it.last) {
+                k1 = k0 + sg.ctl[1];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) load_state<false>(sg, it.at, (uint32_t)(q * 64 + lane), p[q]);
+            }
+        }
 
-        const int nbatch = (int)((maxlast + BATCH - 1) / BATCH);
+        const int nbatch = (int)((k1 - k0 + BATCH - 1) / BATCH);
         for (int b = nbatch - 1; b >= 0; --b) {
-            const uint32_t base = start + (uint32_t)b * BATCH;
-            const uint32_t cnt = min(min((uint32_t)BATCH, end - base), maxlast - (uint32_t)b * BATCH);
+            const uint32_t first_k = k0 + (uint32_t)b * BATCH;
+            const uint32_t base = start + first_k;
+            const uint32_t cnt = min((uint32_t)BATCH, k1 - first_k);
             __syncthreads();  // the previous batch's walk has read its LDS
             uint32_t count = 0;
 #pragma unroll
@@ -512,7 +650,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                     s_a[slot] = r.a_px;
                     s_b[slot] = r.b_py;
                     s_c[slot] = r.col_op;
-                    s_lthr[slot] = record_lthr(r.col_op.w);
                     qmask = cull ? block_mask<16>(r, x0, y0) : 0xFu;
                 }
                 const uint64_t bal = __ballot(qmask != 0u);
@@ -526,7 +663,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                 const uint32_t e = __builtin_amdgcn_readfirstlane((uint32_t)s_list[kk]);
                 const uint32_t j = e & ((1u << MB) - 1u);
                 const uint32_t qm = e >> MB;
-                const uint32_t rel = (uint32_t)b * BATCH + j;
+                const uint32_t rel = first_k + j;
                 bool need[4];
                 bool any_need = false;
 #pragma unroll
@@ -541,7 +678,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                 r.b_py = s_b[j];
                 r.col_op = s_c[j];
                 r.nrm_dep = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                const float lthr = s_lthr[j];
                 float g[16];
                 float g2[4];
                 g[kGNt] = 0.0f;
@@ -549,7 +685,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     if (!need[q]) continue;
-                    const HitEval h = eval_hit(r, p[q].sx, p[q].sy, p[q].pxc, p[q].pyc, lthr);
+                    const HitEval h = eval_hit(r, p[q].sx, p[q].sy, p[q].pxc, p[q].pyc);
                     const bool act = rel < p[q].last && h.alpha > 0.0f;
                     if (!__any(act)) continue;
                     if (first) add_hit<false, false>(p[q], r, h, act, 0.0f, g, g2);
@@ -574,30 +710,191 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
     }
 }
 
+// Clears the gradient accumulator and the split flags, resets the cursors and
+// the segment counter and sets the segment length: one launch per pass.
+__global__ __launch_bounds__(256) void bwd_prepare_kernel(float4* __restrict__ grad_coef, size_t vecs,
+                                                          uint32_t* __restrict__ cursor, BwdSegments sg,
+                                                          uint32_t split_tiles,
+                                                          const uint32_t* __restrict__ entries) {
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+    if (t == 0) {
+        const uint32_t e = *entries;
+        sg.ctl[0] = 0u;
+        sg.ctl[1] = max(kSegmentMin, (e / kSegmentTarget + 31u) / 32u * 32u);
+    }
+    if (cursor != nullptr && t < kTileQueues) cursor[t] = 0u;
+    for (size_t k = t; k < split_tiles; k += step) sg.split[k] = 0u;
+    for (size_t k = t; k < vecs; k += step) grad_coef[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// State pass of the lists longer than a segment (16-px tiles; ctl[1] records
+// per segment): claims the tile's segments, walks the records past the first
+// segment back to front and stores every pixel's walk state at the segment
+// boundaries. The arithmetic per (pixel, record) is the gradient pass's
+// (step_state), so each segment continues with the bits the whole walk would
+// have. A workgroup is four waves, one per 8x8 block; nothing is summed over
+// pixels here, so each 16-lane row walks its own list of the records that
+// reach its 4x4 sub-block: a list is about a third of the tile's, and a
+// record's step has 45 instructions against ~270 with gradients and their
+// reduction, which is what shortens the critical path. 250k surfels at 1283 x
+// 717: 108 us for the state pass and 332 us for the gradient pass, where the
+// gradient pass over whole lists takes 1042 us (its longest list); 200k
+// surfels in six 640 x 360 views: 321 + 811 against 2085 us. Where no list is
+// longer than a segment (1M surfels, four 1080p views) the pass is 5 us.
+template <bool AUX>
+__global__ __launch_bounds__(256) void raster_state_kernel(
+    const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
+    const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in, bool cull,
+    uint32_t total_tiles, TileQueue queue, BwdSegments sg) {
+    constexpr int BATCH = 128;               // records staged at a time, two threads each
+    __shared__ float4 s_rec[4][BATCH];       // M Nt | A px | B py | colour opacity
+    __shared__ float4 s_n[AUX ? BATCH : 1];
+    __shared__ uint8_t s_mask[BATCH][4];     // per sub-block line: the columns the record reaches
+    __shared__ uint8_t s_list[16][BATCH];
+    __shared__ uint32_t s_last[4], s_base;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // Row g of wave w: sub-block (2 (w & 1) + (g & 1), 2 (w >> 1) + (g >> 1)),
+    // lane p its pixel (p & 3, p >> 2).
+    const int g = lane >> 4, p = lane & 15;
+    const int sc = 2 * (wave & 1) + (g & 1), sr = 2 * (wave >> 1) + (g >> 1);
+    const int slot = tid >> 1, part = tid & 1;
+    uint8_t* const my_list = s_list[sr * 4 + sc];
+    // The pixel's index within the stored state: block, then row-major.
+    const uint32_t pixel = (uint32_t)(wave * 64 + ((4 * (g >> 1) + (p >> 2)) * 8 + 4 * (g & 1) + (p & 3)));
+    const uint32_t seg_len = sg.ctl[1];
+    for (uint32_t pos = blockIdx.x; pos < total_tiles; pos += gridDim.x) {
+        const uint32_t gtile = queue.order[pos];
+        const uint32_t start = ranges[2 * (size_t)gtile], end = ranges[2 * (size_t)gtile + 1];
+        // Longest lists first (keys saturate at 0xFFFF): no longer one follows.
+        if (end - start <= min(seg_len, 0xFFFFu)) break;
+        const CamParams& cam = cams[view_of_tile(cams, n_views, gtile)];
+        const uint32_t local = gtile - cam.tile_base;
+        const uint32_t x0 = (local % cam.tiles_x) * 16, y0 = (local / cam.tiles_x) * 16;
+        const float lambda = AUX ? cam.lambda_dist : 0.0f;
+        PixState ps;
+        load_pixel<AUX>(ps, cam, (int)x0 + 4 * sc + (p & 3), (int)y0 + 4 * sr + (p >> 2), in, lambda);
+        uint32_t row_last = ps.last;
+        for (int o = 8; o >= 1; o >>= 1) row_last = max(row_last, (uint32_t)__shfl_xor((int)row_last, o));
+        uint32_t wave_last = row_last;
+        for (int o = 32; o >= 16; o >>= 1) wave_last = max(wave_last, (uint32_t)__shfl_xor((int)wave_last, o));
+        if (lane == 0) s_last[wave] = wave_last;
+        __syncthreads();
+        const uint32_t maxlast =
+            __builtin_amdgcn_readfirstlane(max(max(s_last[0], s_last[1]), max(s_last[2], s_last[3])));
+        const uint32_t nseg = (maxlast + seg_len - 1) / seg_len;
+        if (nseg < 2) {
+            __syncthreads();  // s_last is rewritten by the next tile
+            continue;
+        }
+        if (tid == 0) s_base = atomicAdd(sg.ctl, nseg);
+        __syncthreads();
+        const uint32_t at = __builtin_amdgcn_readfirstlane(s_base);
+        const bool room = at + nseg <= sg.pool;  // by segment_pool always
+        for (uint32_t k = (uint32_t)tid; k < nseg && at + k < sg.pool; k += 256)
+            sg.table[at + k] = make_uint2(room ? gtile : ~0u, k + 1 == nseg ? k | kSegmentLast : k);
+        if (tid == 0 && room) sg.split[gtile] = 1u;
+        if (!room) continue;  // walked whole by the gradient pass
+        for (uint32_t s = nseg - 1; s >= 1; --s) {
+            const uint32_t k0 = s * seg_len, k1 = min(maxlast, k0 + seg_len);
+            const int nbatch = (int)((k1 - k0 + BATCH - 1) / BATCH);
+            for (int b = nbatch - 1; b >= 0; --b) {
+                const uint32_t first = k0 + (uint32_t)b * BATCH;
+                const uint32_t cnt = min((uint32_t)BATCH, k1 - first);
+                __syncthreads();  // the previous walk has read the staged records
+                if ((uint32_t)slot < cnt) {
+                    const Record* src = recs + payloads[start + first + slot];
+                    const float4* f4 = reinterpret_cast<const float4*>(src);
+                    const float4 box = src->box, e0 = src->ell0, e1 = src->ell1;
+                    const float cx = src->a_px.w, cy = src->b_py.w;
+                    s_rec[2 * part][slot] = f4[2 * part];
+                    s_rec[2 * part + 1][slot] = f4[2 * part + 1];
+                    if (AUX && part == 0) s_n[slot] = src->nrm_dep;
+                    const SubTest t = sub_test(box, e0, e1, cx, cy);
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        const int row = 2 * part + r;
+                        s_mask[slot][row] = cull ? (uint8_t)sub_row_mask(t, (float)x0, (float)(y0 + 4 * row)) : 0xFu;
+                    }
+                }
+                __syncthreads();
+                // Each row's list, in batch order: the records that reach its
+                // sub-block before its last contributor.
+                uint32_t count = 0;
+                for (uint32_t k = 0; k < cnt; k += 16) {
+                    const uint32_t j = k + (uint32_t)p;
+                    const bool in_list =
+                        j < cnt && first + j < row_last && ((s_mask[min(j, cnt - 1)][sr] >> sc) & 1u);
+                    const uint32_t bal = (uint32_t)(__ballot(in_list) >> (16 * g)) & 0xFFFFu;
+                    if (in_list) my_list[count + (uint32_t)__popc(bal & ((1u << p) - 1u))] = (uint8_t)j;
+                    count += (uint32_t)__popc(bal);
+                }
+                __builtin_amdgcn_wave_barrier();
+                for (int kk = (int)count - 1; kk >= 0; --kk) {
+                    const uint32_t j = my_list[kk];
+                    Record r;
+                    r.m_nt = s_rec[0][j];
+                    r.a_px = s_rec[1][j];
+                    r.b_py = s_rec[2][j];
+                    r.col_op = s_rec[3][j];
+                    r.nrm_dep = AUX ? s_n[AUX ? j : 0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    const HitEval h = eval_hit(r, ps.sx, ps.sy, ps.pxc, ps.pyc);
+                    step_state<AUX>(ps, r, h, first + j < ps.last && h.alpha > 0.0f, lambda);
+                }
+            }
+            store_state<AUX>(sg, at + s - 1, pixel, ps);
+        }
+        __syncthreads();  // s_last and s_base are rewritten by the next tile
+    }
+}
+
 template <bool AUX, int TW, int BATCH>
 void launch_bwd(hipStream_t st, uint32_t grid, const CamParams* cams_dev, uint32_t n_views,
                 uint32_t total_tiles, const uint32_t* ranges, const uint32_t* payloads, const Record* recs,
-                BwdIn in, float* grad_coef, bool cull, TileQueue queue, uint32_t tile_begin) {
+                BwdIn in, float* grad_coef, bool cull, TileQueue queue, uint32_t tile_begin, BwdSegments sg) {
     constexpr int NT = TW == 8 ? 64 : TW * TW / 2;
     hipLaunchKernelGGL((raster_bwd_kernel<AUX, TW, BATCH>), dim3(grid), dim3(NT), 0, st, cams_dev, n_views,
-                       ranges, payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin);
+                       ranges, payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
 }
 
 }  // namespace
+
+hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
+                              uint32_t split_tiles, const uint32_t* entries) {
+    const size_t vecs = floats / 4;
+    if (floats % 4 != 0) return hipErrorInvalidValue;
+    uint64_t blocks = (std::max<size_t>(vecs, split_tiles) + 255) / 256;
+    blocks = std::min<uint64_t>(std::max<uint64_t>(blocks, 1), 4096);
+    hipLaunchKernelGGL(bwd_prepare_kernel, dim3((uint32_t)blocks), dim3(256), 0, st,
+                       reinterpret_cast<float4*>(grad_coef), vecs, cursor, sg, split_tiles, entries);
+    return hipGetLastError();
+}
 
 hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const CamParams* /*cams_host*/,
                              uint32_t n_views, uint32_t total_tiles, const uint32_t* ranges,
                              const uint32_t* payloads, const Record* recs, BwdIn in,
                              float* grad_coef, bool aux, bool cull, TileQueue queue, RasterShape shape,
-                             uint32_t tile_begin) {
+                             uint32_t tile_begin, BwdSegments sg) {
     if (total_tiles == 0) return hipSuccess;
-    const uint32_t grid = queue.cursor != nullptr ? std::min(total_tiles, std::max(queue.grid_blocks, 1u))
-                                                  : total_tiles;
     const uint32_t t = shape.tile, b = shape.bwd_batch;
+    // Segments need the queue (its order and cursors) and 16-px tiles.
+    if (queue.cursor == nullptr || t != 16) sg = BwdSegments{};
+    const uint32_t most = total_tiles + (sg.state != nullptr ? sg.pool : 0u);
+    const uint32_t grid = queue.cursor != nullptr ? std::min(most, std::max(queue.grid_blocks, 1u)) : total_tiles;
     auto go = [&](auto fn) {
         fn(st, grid, cams_dev, n_views, total_tiles, ranges, payloads, recs, in, grad_coef, cull, queue,
-           tile_begin);
+           tile_begin, sg);
     };
+    if (sg.state != nullptr) {
+        const uint32_t g = std::min(total_tiles, std::max(queue.grid_blocks / 2, 1u));
+        if (aux)
+            hipLaunchKernelGGL(raster_state_kernel<true>, dim3(g), dim3(256), 0, st, cams_dev, n_views, ranges,
+                               payloads, recs, in, cull, total_tiles, queue, sg);
+        else
+            hipLaunchKernelGGL(raster_state_kernel<false>, dim3(g), dim3(256), 0, st, cams_dev, n_views, ranges,
+                               payloads, recs, in, cull, total_tiles, queue, sg);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     if (aux) {
         if (t != 16) return hipErrorInvalidValue;  // depth / normal losses: 16-px tiles
         go(launch_bwd<true, 16, 128>);
@@ -607,14 +904,14 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
         go(launch_bwd<false, 8, 128>);
     } else if (t == 16) {
         // One wave per tile: twice the workgroups for the same waves per CU.
-        const uint32_t g2 = queue.cursor != nullptr ? std::min(total_tiles, std::max(2 * queue.grid_blocks, 1u))
+        const uint32_t g2 = queue.cursor != nullptr ? std::min(most, std::max(2 * queue.grid_blocks, 1u))
                                                     : total_tiles;
         if (b == 64)
             hipLaunchKernelGGL(raster_bwd_wave_kernel<64>, dim3(g2), dim3(64), 0, st, cams_dev, n_views, ranges,
-                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin);
+                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
         else if (b == 128)
             hipLaunchKernelGGL(raster_bwd_wave_kernel<128>, dim3(g2), dim3(64), 0, st, cams_dev, n_views, ranges,
-                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin);
+                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
         else
             return hipErrorInvalidValue;
     } else if (t == 32 && b == 128) {

@@ -9,8 +9,7 @@
 // each record's alpha >= 1/255 footprint (box clipped to its 16-px rect,
 // screen disk and ellipse, computed at projection) is tested against the
 // tile's blocks, and the batch is split into order-preserving per-block
-// lists, so a wave only walks the records that can touch its 64 pixels. Per
-// pixel, an exponent test rejects non-contributing records before exp(). A
+// lists, so a wave only walks the records that can touch its 64 pixels. A
 // wave leaves the batch once its pixels are saturated; the workgroup stops
 // when every pixel's transmittance is below 1e-4.
 //
@@ -55,7 +54,6 @@ __attribute__((amdgpu_waves_per_eu((!AUX && TW == 16) ? 7 : 1))) void raster_fwd
     constexpr int SPT = (BATCH + NT - 1) / NT;  // batch slots per thread
     static_assert(BATCH % 64 == 0 && BATCH <= 1024, "batch of whole waves");
     __shared__ float4 s_m[BATCH], s_a[BATCH], s_b[BATCH], s_c[BATCH], s_n[AUX ? BATCH : 1];
-    __shared__ float s_lthr[BATCH];
     __shared__ uint16_t s_list[NB][BATCH];
     __shared__ uint32_t s_qcnt[SW][NB];
     __shared__ uint32_t s_view, s_next;
@@ -121,7 +119,6 @@ __attribute__((amdgpu_waves_per_eu((!AUX && TW == 16) ? 7 : 1))) void raster_fwd
                     s_b[slot] = r.b_py;
                     s_c[slot] = r.col_op;
                     if (AUX) s_n[slot] = r.nrm_dep;
-                    s_lthr[slot] = record_lthr(r.col_op.w);
                     qm[m] = cull ? block_mask<TW>(r, x0, y0) : all_blocks;
                 }
                 // Order-preserving split of the batch into per-block lists.
@@ -153,16 +150,15 @@ __attribute__((amdgpu_waves_per_eu((!AUX && TW == 16) ? 7 : 1))) void raster_fwd
             for (int w = 0; w < SW; ++w) my_count += s_qcnt[w][wave];
             __syncthreads();
             if (__any(T >= kTTerminate)) {
-                auto load = [&](uint32_t j, Record& r, float& lthr) {
+                auto load = [&](uint32_t j, Record& r) {
                     r.m_nt = s_m[j];
                     r.a_px = s_a[j];
                     r.b_py = s_b[j];
                     r.col_op = s_c[j];
                     r.nrm_dep = AUX ? s_n[AUX ? j : 0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    lthr = s_lthr[j];
                 };
-                auto composite = [&](uint32_t j, const Record& r, float lthr) {
-                    const HitEval h = eval_hit(r, sx, sy, pxc, pyc, lthr);
+                auto composite = [&](uint32_t j, const Record& r) {
+                    const HitEval h = eval_hit(r, sx, sy, pxc, pyc);
                     if (T >= kTTerminate && h.alpha > 0.0f) {
                         const float w = T * h.alpha;
                         cr += r.col_op.x * w;
@@ -195,14 +191,13 @@ __attribute__((amdgpu_waves_per_eu((!AUX && TW == 16) ? 7 : 1))) void raster_fwd
                     const uint32_t j0 = s_list[wave][k];
                     const uint32_t j1 = two ? (uint32_t)s_list[wave][k + 1] : j0;
                     Record r0, r1;
-                    float l0, l1;
-                    load(j0, r0, l0);
-                    load(j1, r1, l1);
+                    load(j0, r0);
+                    load(j1, r1);
                     // One saturation test per round: a wave done after j0
                     // walks j1 with every lane masked off (no contribution).
-                    composite(j0, r0, l0);
+                    composite(j0, r0);
                     if (!two) break;
-                    composite(j1, r1, l1);
+                    composite(j1, r1);
                     if (!__any(T >= kTTerminate)) break;
                 }
             }

@@ -52,13 +52,18 @@ gs_status hip_fail(hipError_t e, const char* what) {
 
 // --------------------------------------------------------------- allocation
 
+// zero = false: scratch that every pass writes before it reads.
 template <typename T>
-static gs_status dalloc(T** out, size_t count, const char* what) {
+static gs_status dalloc(T** out, size_t count, const char* what, bool zero = true) {
     *out = nullptr;
     if (count == 0) count = 1;
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, count * sizeof(T));
     if (e != hipSuccess) return hip_fail(e, what);
+    if (!zero) {
+        *out = static_cast<T*>(p);
+        return GS_OK;
+    }
     // The zero fill runs on the null stream, which is not ordered with the
     // context's non-blocking stream: wait for it, or a kernel enqueued right
     // after the allocation can be overwritten by the late fill.
@@ -597,6 +602,7 @@ struct RasterCore {
     uint32_t* ncontrib = nullptr;
     float* grad_coef = nullptr;
     float* cam_partials = nullptr;
+    BwdSegments segs;                // long lists of the backward, split over depth
     // Decision trace of the forward (verification aid; lists == nullptr: off).
     FwdTrace trace;
     // Depth-presort path (binning = GS_BINNING_PRESORT or GS_BINNING_TIGHT).
@@ -654,6 +660,10 @@ struct RasterCore {
         dfree(ncontrib);
         dfree(grad_coef);
         dfree(cam_partials);
+        dfree(segs.ctl);
+        dfree(segs.table);
+        dfree(segs.split);
+        dfree(segs.state);
         for (int i = 0; i < 2; ++i) {
             dfree(pre_keys[i]);
             dfree(pre_vals[i]);
@@ -669,8 +679,10 @@ struct RasterCore {
         dfree(cursors);
     }
 
+    // aux: backward passes with depth / normal losses may run (their segment
+    // states hold three vectors per pixel instead of one).
     gs_status init(gs_ctx c, uint32_t n, uint32_t views, uint32_t entries, uint32_t tiles,
-                   uint32_t pixels) {
+                   uint32_t pixels, bool aux) {
         ctx = c;
         if (entries >= (1u << 30)) return fail(GS_ERR_CAPACITY, "max_entries must be < 2^30");
         if ((uint64_t)n * views >= (1ull << 32)) return fail(GS_ERR_CAPACITY, "views * surfels must be < 2^32");
@@ -732,6 +744,12 @@ struct RasterCore {
         GS_CHECK(dalloc(&out_normal, pixels, "out_normal"));
         GS_CHECK(dalloc(&ncontrib, pixels, "ncontrib"));
         GS_CHECK(dalloc(&grad_coef, nv * kGradStride, "grad_coef"));
+        segs.pool = segment_pool(entries);
+        GS_CHECK(dalloc(&segs.ctl, 2, "segment control"));
+        GS_CHECK(dalloc(&segs.table, segs.pool, "segment table"));
+        GS_CHECK(dalloc(&segs.split, tiles, "split tiles"));
+        GS_CHECK(dalloc(&segs.state, (size_t)segs.pool * kSegmentPixels * (aux ? 3 : 1), "segment states",
+                        false));
         uint8_t* cp = nullptr;
         GS_CHECK(dalloc(&cp, geom_cam_partials_bytes(n, views), "camera partials"));
         cam_partials = reinterpret_cast<float*>(cp);
@@ -942,14 +960,13 @@ struct RasterCore {
         uint32_t tiles = 0;
         for (uint32_t v = v0; v < v0 + nv; ++v) tiles += cams[v].tiles_x * cams[v].tiles_y;
         GS_CHECK(P.mark(st, GS_STAGE_GRAD_CLEAR));
-        GS_HIP(launch_fill_u32(st, reinterpret_cast<uint32_t*>(grad_coef), 0u,
-                               (size_t)n * nv * grad_stride(aux)));
         BwdIn in{dl_dcolor, dl_dnormal, out_color, out_aux, ncontrib};
-        GS_CHECK(P.mark(st, GS_STAGE_RASTER_BWD));
         const TileQueue qb = (q_tiles[0] == tiles && q_begin[0] == 0) ? queue(0, 1) : TileQueue{nullptr, nullptr, 0};
-        if (qb.cursor != nullptr) GS_HIP(launch_fill_u32(st, qb.cursor, 0u, kTileQueues));
+        GS_HIP(launch_bwd_prepare(st, grad_coef, (size_t)n * nv * grad_stride(aux), qb.cursor, segs, tiles,
+                                  last_sort_count));
+        GS_CHECK(P.mark(st, GS_STAGE_RASTER_BWD));
         GS_HIP(launch_raster_bwd(st, cd, cams.data() + v0, nv, tiles, ranges, pays[result_alt], recs, in,
-                                 grad_coef, aux, cull, qb, shape));
+                                 grad_coef, aux, cull, qb, shape, 0, segs));
         if (!geom) return GS_OK;
         GS_CHECK(P.mark(st, GS_STAGE_GEOM_BWD));
         GS_HIP(launch_geom_bwd(st, cd, nv, n, pos, sc, q, sh, grad_coef, aux, g, accumulate,
@@ -1051,7 +1068,7 @@ gs_status gs_raster_create_batch(gs_ctx ctx, uint32_t capacity, uint32_t width, 
     r->max_views = max_views;
     const uint32_t tiles = div_up(width, kTile) * div_up(height, kTile);
     const uint32_t px = width * height * max_views;
-    GS_CHECK(r->core.init(ctx, capacity, max_views, max_entries * max_views, tiles * max_views, px));
+    GS_CHECK(r->core.init(ctx, capacity, max_views, max_entries * max_views, tiles * max_views, px, true));
     GS_CHECK(dalloc(&r->positions, capacity, "positions"));
     GS_CHECK(dalloc(&r->scales, capacity, "scales"));
     GS_CHECK(dalloc(&r->quats, capacity, "quats"));
@@ -2440,7 +2457,7 @@ gs_status gs_trainer_create(gs_ctx ctx, const gs_train_config* cfg, const gs_sce
     const uint64_t per_view_entries = cfg->entries_per_view ? cfg->entries_per_view : (uint64_t)n * 64;
     const uint64_t entries = per_view_entries * V;
     if (entries >= (1ull << 30)) return fail(GS_ERR_CAPACITY, "entries per step must be < 2^30");
-    GS_CHECK(t->core.init(ctx, n, V, (uint32_t)entries, max_tiles * V, max_px * V));
+    GS_CHECK(t->core.init(ctx, n, V, (uint32_t)entries, max_tiles * V, max_px * V, false));
     t->core.digit_bits = cfg->digit_bits ? cfg->digit_bits : 8;
     t->core.binning = cfg->binning;
     // The step's losses are colour-only (L1 + D-SSIM): the forward skips the
