@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void tile_order_keys_kernel(const uint32_t* __
                                                               uint32_t* __restrict__ cursors) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) *count = total_tiles;
-    if (t < 2 * kTileQueues) cursors[t] = 0u;
+    if (t < 2 * kTileQueues) cursors[t * kCursorStride] = 0u;
     if (t >= total_tiles) return;
     const size_t g = (size_t)tile_begin + t;
     const uint32_t len = ranges[2 * g + 1] - ranges[2 * g];
@@ -351,7 +351,7 @@ hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_
 hipError_t launch_tile_order_keys(hipStream_t st, const uint32_t* ranges, uint32_t tile_begin,
                                   uint32_t total_tiles, uint32_t* keys, uint32_t* vals, uint32_t* count,
                                   uint32_t* cursors) {
-    const uint32_t blocks = div_up(total_tiles > 0 ? total_tiles : 1, 256);
+    const uint32_t blocks = div_up(std::max(total_tiles, 2 * kTileQueues), 256);
     hipLaunchKernelGGL(tile_order_keys_kernel, dim3(blocks), dim3(256), 0, st, ranges, tile_begin, total_tiles,
                        keys, vals, count, cursors);
     return hipGetLastError();

@@ -678,16 +678,22 @@ struct FwdTrace {
 };
 constexpr uint32_t kTraceRecordMask = (1u << 30) - 1u;
 // Tile scheduling for the raster passes: with a queue (cursor != nullptr),
-// grid_blocks resident workgroups pull tile positions from kTileQueues
-// cursors (which must be 0 at launch): workgroup b uses cursor
-// x = b % q, q = min(kTileQueues, grid), and claim j of it is position
-// k = j q + x; the workgroup processes tile order[k] (longest list first)
-// until k >= total_tiles. Several cursors spread the atomics over several
-// addresses. Without a queue, workgroup b processes tile b.
-constexpr uint32_t kTileQueues = 8;
+// grid_blocks resident workgroups work through the positions of order[]
+// (longest list first): workgroup b starts with position b, then claims from
+// one of kTileQueues cursors (which must be 0 at launch): workgroup b uses
+// cursor x = b % q, q = min(kTileQueues, grid), and claim j of it is position
+// grid + j q + x, until that passes the last. Without a queue, workgroup b
+// processes tile b. A claim is an atomic at the memory side, 11.4 ns apart for
+// cursors that share a 64-B line (47 us until 4096 workgroups had their first,
+// 0.66 ms for the 57600 tiles of sixteen 720p views), so the first position
+// needs none and the cursors are kCursorStride words apart (0.26 ns with 64 of
+// them, 1.9 ns with 8).
+constexpr uint32_t kTileQueues = 64;
+constexpr uint32_t kCursorStride = 64;
+constexpr uint32_t kCursorWords = kTileQueues * kCursorStride;  // one set of cursors
 struct TileQueue {
     const uint32_t* order;
-    uint32_t* cursor;  // kTileQueues counters
+    uint32_t* cursor;  // kTileQueues counters, kCursorStride words apart
     uint32_t grid_blocks;
 };
 // Work-tile size (px; must equal every view's CamParams::tile_size) and the
@@ -702,6 +708,11 @@ struct RasterShape {
     uint32_t fwd_batch = 256;
     uint32_t bwd_batch = 64;
 };
+// Position of workgroup blockIdx.x's next claim (one lane).
+__device__ __forceinline__ uint32_t claim_position(const TileQueue& queue) {
+    const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
+    return gridDim.x + atomicAdd(queue.cursor + x * kCursorStride, 1u) * q + x;
+}
 // The pass covers total_tiles tiles: queue.order[0 .. total_tiles) with a
 // queue, else the global tiles [tile_begin, tile_begin + total_tiles).
 hipError_t launch_raster_fwd(hipStream_t st, const CamParams* cams_dev, const CamParams* cams_host,
@@ -727,7 +738,8 @@ struct BwdIn {
 // launch's critical path. state == nullptr: off.
 constexpr uint32_t kSegmentPool = 12288;   // segments of one pass
 constexpr uint32_t kSegmentTarget = 6144;  // a segment holds at least 1 / this of the entries
-constexpr uint32_t kSegmentMin = 32;       // and at least this many records
+constexpr uint32_t kSegmentMin = 32;       // and at least this many records,
+constexpr uint32_t kSegmentMinAux = 64;    // with aux, whose states are three times as large
 constexpr uint32_t kSegmentPixels = 256;
 constexpr uint32_t kSegmentLast = 1u << 31;
 struct BwdSegments {
@@ -739,7 +751,11 @@ struct BwdSegments {
 };
 // Split tiles' lists are longer than a segment of at least E / kSegmentTarget
 // (E = entries) and at least kSegmentMin records, so a tile has at most 2 len
-// / L of them and all have at most 2 E / L.
+// / L of them and all have at most 2 E / L. Measured at 6144 and 32 against
+// half and twice the target: plain 250k 2x1283x717 1738 against 1827 / 1732 us,
+// batch 200k 6x640x360 1857 against 1965 / 1815 us, 100k eight uneven views 1557
+// against 1558 / 1642 us; a minimum of 64 loses 3 % at 10k 256px (396 against
+// 384 us) and gains 9 % with aux (20k 321x243: 483 against 531 us).
 constexpr uint32_t segment_pool(uint32_t max_entries) {
     const uint64_t most = 2ull * max_entries / kSegmentMin + 16;
     return (uint32_t)(most < kSegmentPool + 16 ? most : kSegmentPool + 16);
@@ -748,7 +764,7 @@ constexpr uint32_t segment_pool(uint32_t max_entries) {
 // backward pass: the queue's cursors (optional), the split flags of
 // split_tiles tiles and the segment length for *entries entries.
 hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
-                              uint32_t split_tiles, const uint32_t* entries);
+                              uint32_t split_tiles, const uint32_t* entries, bool aux);
 hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const CamParams* cams_host,
                              uint32_t n_views, uint32_t total_tiles, const uint32_t* ranges,
                              const uint32_t* payloads, const Record* recs, BwdIn in,

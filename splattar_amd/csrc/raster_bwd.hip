@@ -151,21 +151,22 @@ __device__ __forceinline__ void load_pixel(PixState& p, const CamParams& cam, in
     p.last = has_loss ? last : 0u;
 }
 
-// The walk state's own arithmetic is written with explicit fmaf: the state
-// pass (raster_state_kernel) has to reach the gradient pass's values bit for
-// bit, which contraction left to the compiler would not promise.
-// d(distortion)/dw of a hit and, in dt_dist, its derivative with respect to
-// the hit's depth (backward.rs:126-153).
+// The walk state's own arithmetic, shared by the gradient pass (add_hit) and
+// the state pass (step_state), which has to reach the same bits: every
+// multiply-add is explicit, nothing is left to contraction.
+// Derivative of the distortion with respect to a hit's weight and, in
+// dt_dist, its depth (backward.rs:126-153); lambda != 0.
 __device__ __forceinline__ float distortion_coef(const PixState& p, float w, float t_hit, float lambda,
                                                  float& dt_dist) {
-    if (lambda == 0.0f) return 0.0f;
+#pragma clang fp contract(off)
     const float a_pre = p.w_total - p.suf_w - w;
     const float b_pre = fmaf(-w, t_hit, p.wt_total - p.suf_d);
     dt_dist = lambda * 2.0f * w * (a_pre - p.suf_w);
     return lambda * fmaf(2.0f, fmaf(t_hit, a_pre, -b_pre), 2.0f * fmaf(-t_hit, p.suf_w, p.suf_d));
 }
 __device__ __forceinline__ void step_aux_sums(PixState& p, const Record& r, float w, float t_hit, float coef) {
-    p.suf_d = fmaf(t_hit, w, p.suf_d);
+#pragma clang fp contract(off)
+    p.suf_d += t_hit * w;
     p.suf_nx = fmaf(r.nrm_dep.x, w, p.suf_nx);
     p.suf_ny = fmaf(r.nrm_dep.y, w, p.suf_ny);
     p.suf_nz = fmaf(r.nrm_dep.z, w, p.suf_nz);
@@ -183,8 +184,8 @@ __device__ __forceinline__ void step_state(PixState& p, const Record& r, const H
     p.suf_g = fmaf(r.col_op.y, w, p.suf_g);
     p.suf_b = fmaf(r.col_op.z, w, p.suf_b);
     if (AUX) {
-        float dt_dist = 0.0f;
-        const float coef = distortion_coef(p, w, h.t, lambda, dt_dist);
+        float dt_dist = 0.0f, coef = 0.0f;
+        if (lambda != 0.0f) coef = distortion_coef(p, w, h.t, lambda, dt_dist);
         step_aux_sums(p, r, w, h.t, coef);
     }
     p.T = t_before;
@@ -279,8 +280,8 @@ __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitE
     p.suf_g = fmaf(r.col_op.y, w, p.suf_g);
     p.suf_b = fmaf(r.col_op.z, w, p.suf_b);
     if (AUX) {
-        float dt_dist = 0.0f;
-        const float coef = distortion_coef(p, w, t_hit, lambda, dt_dist);
+        float dt_dist = 0.0f, coef = 0.0f;
+        if (lambda != 0.0f) coef = distortion_coef(p, w, t_hit, lambda, dt_dist);
         put<AUX, ACC>(g2[kGNrm - 16 + 0], p.dnx * w);
         put<AUX, ACC>(g2[kGNrm - 16 + 1], p.dny * w);
         put<AUX, ACC>(g2[kGNrm - 16 + 2], p.dnz * w);
@@ -362,20 +363,17 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     const int col = wave % NC, hrow = wave / NC;
     const uint32_t nseg = sg.state != nullptr ? min(sg.ctl[0], sg.pool) : 0u;
     const uint32_t items = total_tiles + nseg;
-    // Room for every item: each workgroup takes one, without a claim.
-    const bool claim = queue.cursor != nullptr && items > gridDim.x;
     for (uint32_t iter = 0;; ++iter) {
         uint32_t pos;
-        if (claim) {
-            if (tid == 0) {
-                const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
-                s_next = atomicAdd(queue.cursor + x, 1u) * q + x;
-            }
+        if (iter == 0) {
+            pos = queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+        } else if (queue.cursor != nullptr) {
+            if (tid == 0) s_next = claim_position(queue);
             __syncthreads();
             pos = s_next;
             __syncthreads();  // every thread has pos before s_next is rewritten
         } else {
-            pos = iter > 0 ? items : queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+            pos = items;
         }
         if (pos >= items) break;
         BwdItem it;
@@ -584,19 +582,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const uint32_t nseg = sg.state != nullptr ? min(sg.ctl[0], sg.pool) : 0u;
     const uint32_t items = total_tiles + nseg;
-    // Room for every item: each wave takes one, without a claim.
-    const bool claims = queue.cursor != nullptr && items > gridDim.x;
     for (uint32_t iter = 0;; ++iter) {
         uint32_t pos;
-        if (claims) {
-            uint32_t claim = 0;
-            if (lane == 0) {
-                const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
-                claim = atomicAdd(queue.cursor + x, 1u) * q + x;
-            }
-            pos = __builtin_amdgcn_readfirstlane(claim);
+        if (iter == 0) {
+            pos = queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+        } else if (queue.cursor != nullptr) {
+            pos = __builtin_amdgcn_readfirstlane(lane == 0 ? claim_position(queue) : 0u);
         } else {
-            pos = iter > 0 ? items : queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+            pos = items;
         }
         if (pos >= items) break;
         BwdItem it;
@@ -715,14 +708,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(float4* __restrict__ grad_coef, size_t vecs,
                                                           uint32_t* __restrict__ cursor, BwdSegments sg,
                                                           uint32_t split_tiles,
-                                                          const uint32_t* __restrict__ entries) {
+                                                          const uint32_t* __restrict__ entries,
+                                                          uint32_t min_len) {
     const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
     if (t == 0) {
         const uint32_t e = *entries;
         sg.ctl[0] = 0u;
-        sg.ctl[1] = max(kSegmentMin, (e / kSegmentTarget + 31u) / 32u * 32u);
+        sg.ctl[1] = max(min_len, (e / kSegmentTarget + 31u) / 32u * 32u);
     }
-    if (cursor != nullptr && t < kTileQueues) cursor[t] = 0u;
+    if (cursor != nullptr && t < kTileQueues) cursor[t * kCursorStride] = 0u;
     for (size_t k = t; k < split_tiles; k += step) sg.split[k] = 0u;
     for (size_t k = t; k < vecs; k += step) grad_coef[k] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
@@ -859,13 +853,14 @@ void launch_bwd(hipStream_t st, uint32_t grid, const CamParams* cams_dev, uint32
 }  // namespace
 
 hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
-                              uint32_t split_tiles, const uint32_t* entries) {
+                              uint32_t split_tiles, const uint32_t* entries, bool aux) {
     const size_t vecs = floats / 4;
     if (floats % 4 != 0) return hipErrorInvalidValue;
     uint64_t blocks = (std::max<size_t>(vecs, split_tiles) + 255) / 256;
     blocks = std::min<uint64_t>(std::max<uint64_t>(blocks, 1), 4096);
     hipLaunchKernelGGL(bwd_prepare_kernel, dim3((uint32_t)blocks), dim3(256), 0, st,
-                       reinterpret_cast<float4*>(grad_coef), vecs, cursor, sg, split_tiles, entries);
+                       reinterpret_cast<float4*>(grad_coef), vecs, cursor, sg, split_tiles, entries,
+                       aux ? kSegmentMinAux : kSegmentMin);
     return hipGetLastError();
 }
 

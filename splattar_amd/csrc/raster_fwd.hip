@@ -62,16 +62,15 @@ __attribute__((amdgpu_waves_per_eu((!AUX && TW == 16) ? 7 : 1))) void raster_fwd
     const uint32_t all_blocks = NB == 32 ? ~0u : (1u << NB) - 1u;
     for (uint32_t iter = 0;; ++iter) {
         uint32_t pos;
-        if (queue.cursor != nullptr) {
-            if (tid == 0) {
-                const uint32_t q = min(kTileQueues, gridDim.x), x = blockIdx.x % q;
-                s_next = atomicAdd(queue.cursor + x, 1u) * q + x;
-            }
+        if (iter == 0) {
+            pos = queue.cursor != nullptr ? blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+        } else if (queue.cursor != nullptr) {
+            if (tid == 0) s_next = claim_position(queue);
             __syncthreads();
             pos = s_next;
             __syncthreads();  // every thread has pos before s_next is rewritten
         } else {
-            pos = iter == 0 ? xcd_swizzle(blockIdx.x, gridDim.x) : total_tiles;
+            pos = total_tiles;
         }
         if (pos >= total_tiles) break;
         const uint32_t gtile = queue.order != nullptr ? queue.order[pos] : tile_begin + pos;

@@ -722,7 +722,7 @@ struct RasterCore {
             GS_CHECK(dalloc(&order_vals[i], tiles ? tiles : 1, "tile order"));
         }
         GS_CHECK(dalloc(&order_count, kRanges, "tile order count"));
-        GS_CHECK(dalloc(&cursors, 2 * kRanges * kTileQueues, "tile cursors"));
+        GS_CHECK(dalloc(&cursors, 2 * kRanges * kCursorWords, "tile cursors"));
         {
             // Persistent raster launches: 8 workgroups per CU (more than can
             // be resident; the rest start as slots free up). GS_TILE_QUEUE=0
@@ -913,7 +913,7 @@ struct RasterCore {
         q_tiles[slot] = 0;
         if (!tile_queue || nt == 0) return GS_OK;
         GS_HIP(launch_tile_order_keys(st, ranges, t0, nt, order_keys[0] + t0, order_vals[0] + t0,
-                                      order_count + slot, cursors + 2 * slot * kTileQueues));
+                                      order_count + slot, cursors + 2 * slot * kCursorWords));
         int alt = 0;
         GS_HIP(launch_radix_sort_u32(st, order_keys[0] + t0, order_vals[0] + t0, order_keys[1] + t0,
                                      order_vals[1] + t0, order_count + slot, nt, 0, 16, 8, sort_scratch, &alt));
@@ -926,7 +926,7 @@ struct RasterCore {
     // 1 = backward cursor set), or none.
     TileQueue queue(int slot, int which) const {
         if (q_tiles[slot] == 0) return TileQueue{nullptr, nullptr, 0};
-        return TileQueue{order_vals[0] + q_begin[slot], cursors + (2 * slot + which) * kTileQueues, queue_blocks};
+        return TileQueue{order_vals[0] + q_begin[slot], cursors + (2 * slot + which) * kCursorWords, queue_blocks};
     }
 
     // Raster passes over the binned tiles [t0, t0 + nt) of views
@@ -944,7 +944,7 @@ struct RasterCore {
         BwdIn in{dl_dcolor, nullptr, out_color, out_aux, ncontrib};
         const TileQueue qb = (q_tiles[slot] == nt && q_begin[slot] == t0) ? queue(slot, 1)
                                                                             : TileQueue{nullptr, nullptr, 0};
-        if (qb.cursor != nullptr) GS_HIP(launch_fill_u32(st, qb.cursor, 0u, kTileQueues));
+        if (qb.cursor != nullptr) GS_HIP(launch_fill_u32(st, qb.cursor, 0u, kCursorWords));
         GS_HIP(launch_raster_bwd(st, cams_dev + v0, cams.data() + v0, nv, nt, ranges, pays[result_alt], recs, in,
                                  grad_coef, false, cull, qb, shape, t0));
         return GS_OK;
@@ -963,7 +963,7 @@ struct RasterCore {
         BwdIn in{dl_dcolor, dl_dnormal, out_color, out_aux, ncontrib};
         const TileQueue qb = (q_tiles[0] == tiles && q_begin[0] == 0) ? queue(0, 1) : TileQueue{nullptr, nullptr, 0};
         GS_HIP(launch_bwd_prepare(st, grad_coef, (size_t)n * nv * grad_stride(aux), qb.cursor, segs, tiles,
-                                  last_sort_count));
+                                  last_sort_count, aux));
         GS_CHECK(P.mark(st, GS_STAGE_RASTER_BWD));
         GS_HIP(launch_raster_bwd(st, cd, cams.data() + v0, nv, tiles, ranges, pays[result_alt], recs, in,
                                  grad_coef, aux, cull, qb, shape, 0, segs));
