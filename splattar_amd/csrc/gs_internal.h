@@ -288,6 +288,8 @@ struct HitEval {
     float inv_d;     // 1 / D (ray branch)
     float uv2;       // u^2 + v^2
     float raw;       // o * ghat
+    float a;         // min(o * ghat, 0.995)
+    bool hit;        // a >= 1/255
     bool ray;
     bool clamped;    // o * ghat > 0.995
 };
@@ -566,13 +568,14 @@ __device__ __forceinline__ HitEval eval_hit(const Record& r, float sx, float sy,
     const float dx = pxc - r.a_px.w, dy = pyc - r.b_py.w;
     const float e_scr = -fmaf(dx, dx, dy * dy);   // 2 sigma^2 = 1 (LOWPASS_SIGMA2 = 0.5)
     h.ray = e_ray >= e_scr;
-    const float e = h.ray ? e_ray : e_scr;
+    const float e = fmaxf(e_ray, e_scr);
     if (!h.ray) h.t = r.nrm_dep.w;
     h.ghat = __expf(e);
     h.raw = r.col_op.w * h.ghat;
     h.clamped = h.raw > kAlphaClamp;
-    float a = fminf(h.raw, kAlphaClamp);
-    h.alpha = a < kAlphaSkip ? 0.0f : a;
+    h.a = fminf(h.raw, kAlphaClamp);
+    h.hit = h.a >= kAlphaSkip;
+    h.alpha = h.hit ? h.a : 0.0f;
     return h;
 }
 
@@ -706,6 +709,7 @@ struct TileQueue {
     const uint32_t* order;
     uint32_t* cursor;  // kTileQueues counters, kCursorStride words apart
     uint32_t grid_blocks;
+    uint32_t cus = 0;  // compute units
 };
 // Work-tile size (px; must equal every view's CamParams::tile_size) and the
 // records staged through LDS per batch by the forward and backward kernels.

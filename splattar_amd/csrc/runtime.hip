@@ -619,6 +619,7 @@ struct RasterCore {
     uint32_t* cursors = nullptr;      // per tile range: forward, backward cursor sets
     bool tile_queue = true;
     uint32_t queue_blocks = 0;       // resident workgroups of a persistent raster launch
+    uint32_t cus = 0;                // compute units of the device
     // Tile ranges scheduled by the last forward: range s covers global tiles
     // [q_begin[s], q_begin[s] + q_tiles[s]) (q_tiles 0: no queue).
     static constexpr int kRanges = 2;
@@ -724,12 +725,13 @@ struct RasterCore {
         GS_CHECK(dalloc(&order_count, kRanges, "tile order count"));
         GS_CHECK(dalloc(&cursors, 2 * kRanges * kCursorWords, "tile cursors"));
         {
-            // Persistent raster launches: 8 workgroups per CU (more than can
-            // be resident; the rest start as slots free up). GS_TILE_QUEUE=0
+            // Persistent raster launches: up to 8 workgroups per CU (the
+            // forward takes what is resident). GS_TILE_QUEUE=0
             // selects one workgroup per tile in tile order instead.
             const char* env = std::getenv("GS_TILE_QUEUE");
             tile_queue = !(env != nullptr && env[0] == '0');
-            queue_blocks = 8u * (uint32_t)std::max(1, ctx->props.multiProcessorCount);
+            cus = (uint32_t)std::max(1, ctx->props.multiProcessorCount);
+            queue_blocks = 8u * cus;
         }
         for (int i = 0; i < 2; ++i) {
             GS_CHECK(dalloc(&pre_keys[i], nv, "presort keys"));
@@ -926,7 +928,7 @@ struct RasterCore {
     // 1 = backward cursor set), or none.
     TileQueue queue(int slot, int which) const {
         if (q_tiles[slot] == 0) return TileQueue{nullptr, nullptr, 0};
-        return TileQueue{order_vals[0] + q_begin[slot], cursors + (2 * slot + which) * kCursorWords, queue_blocks};
+        return TileQueue{order_vals[0] + q_begin[slot], cursors + (2 * slot + which) * kCursorWords, queue_blocks, cus};
     }
 
     // Raster passes over the binned tiles [t0, t0 + nt) of views
