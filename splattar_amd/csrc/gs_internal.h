@@ -805,9 +805,9 @@ hipError_t launch_geom_bwd(hipStream_t st, const CamParams* cams_dev, uint32_t n
 // loss.hip
 // With `view` set, the target is read at target + view->target_base (the
 // per-view descriptor lives in device memory, so a captured graph replays
-// with whatever views the descriptor table holds). partial_sums receives
-// l1_ssim_partials(w, h) pairs (sum |x - y|, sum SSIM); dl_out may be null
-// (loss only). tstats, when set, holds the target's window mean and second
+// with whatever views the descriptor table holds). partial_sums, room for
+// l1_ssim_partials(w, h) pairs, receives the number of sums and as many pairs
+// (sum |x - y|, sum SSIM) after that pair; dl_out may be null (loss only). tstats, when set, holds the target's window mean and second
 // moment per channel (launch_target_stats), at (target pixel) * 3 + channel
 // from the same base offset as the target.
 hipError_t launch_l1_ssim(hipStream_t st, uint32_t w, uint32_t h, float lambda, float dssim_scale,

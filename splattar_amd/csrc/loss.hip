@@ -14,6 +14,7 @@
 // the step then blurs three statistics of the image instead of five).
 #include "gs_internal.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace gs {
@@ -34,7 +35,7 @@ __device__ __forceinline__ float tap(int d) { return c_w[d < 0 ? -d : d]; }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One launch covers the views of a step. A workgroup
-// owns a strip of kSW output columns and SH output rows of one view (all
+// owns a strip of kSW output columns and lv.rows output rows of one view (all
 // three channels) and walks its input rows top to bottom, one row per step:
 //   load    the input row (kSW + 20 pixels: the blur of the coefficient maps
 //           needs them 5 px beyond the strip, and those need 5 px more) as
@@ -66,6 +67,7 @@ struct LossViews {
     uint32_t n;                          // views in this launch
     uint32_t first;                      // view slot of the first (camera table, partials)
     uint32_t partials_stride;            // partial-sum pairs per view slot
+    uint32_t rows;                       // output rows per band
     uint32_t block_begin[kMaxLossViews + 1];
     uint32_t w[kMaxLossViews], h[kMaxLossViews], pix_base[kMaxLossViews];
     float dw[kMaxLossViews], l1w[kMaxLossViews];
@@ -77,7 +79,7 @@ struct LossViews {
 // hides the row barrier better than the third's spare registers would. The
 // TS variant (register rings of 66) is held to that; the other (rings of
 // 88) fits it too when left a looser bound (forced, it spills two).
-template <int SH, bool TS>
+template <bool TS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS ? 4 : 3))) void l1_ssim_fused_kernel(
     LossViews lv, const float4* __restrict__ img_base, const float4* __restrict__ tgt_base,
     float4* __restrict__ dl_base, double* __restrict__ partials, const CamParams* __restrict__ cams,
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS ? 4 : 3)
     const uint32_t tbase = cams != nullptr ? cams[lv.first + v].target_base : 0u;
     const float4* tgt = tgt_base + tbase;
     const uint32_t strips = (W + kSW - 1) / kSW;
-    const int x0 = (int)(blk % strips) * kSW, y0 = (int)(blk / strips) * SH;
+    const int sh = (int)lv.rows, x0 = (int)(blk % strips) * kSW, y0 = (int)(blk / strips) * sh;
     const int iW = (int)W, iH = (int)H;
     // Stats role: thread 3 cA + chA is (stat column x0 - 5 + cA, channel chA);
     // output role: thread 3 cB + chB is (output column x0 + cB, channel chB).
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS ? 4 : 3)
     const bool colB_in = roleB && gxB < iW;
     float ra[11][NR], rb[11][3];
     double l1 = 0.0, ss = 0.0;
-    constexpr int nrows = SH + 4 * kH;  // input rows y0 - 10 .. y0 + SH + 9
+    const int nrows = min(sh, iH - y0) + 4 * kH;  // input rows from y0 - 10 on
     // Step i (0 <= i <= nrows): input row y0 - 10 + i and stat row
     // y0 - 15 + i (i < nrows); the C-map row of the previous step's stat row
     // is blurred horizontally and output row y0 - 21 + i is finished. In the
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS ? 4 : 3)
                     cm = ds_dmux * dw;
                     cx2 = (-l * cs * rq) * dw;
                     cxy = (2.0f * l * rq) * dw;
-                    if (colA_own && sy >= y0 && sy < y0 + SH) ss += (double)(l * cs);
+                    if (colA_own && sy >= y0 && sy < y0 + sh) ss += (double)(l * cs);
                 }
             }
         }
@@ -324,24 +326,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS ? 4 : 3)
     }
     __syncthreads();
     if (tid == 0) {
-        double* pp = partials + ((size_t)(lv.first + v) * lv.partials_stride + blk) * 2;
+        double* slot = partials + (size_t)(lv.first + v) * lv.partials_stride * 2;
+        if (blk == 0) slot[0] = (double)(lv.block_begin[v + 1] - lv.block_begin[v]);
+        double* pp = slot + 2 * (blk + 1);
         pp[0] = ((s_red[0][0] + s_red[0][1]) + s_red[0][2]) + s_red[0][3];
         pp[1] = ((s_red[1][0] + s_red[1][1]) + s_red[1][2]) + s_red[1][3];
     }
 }
 
-constexpr uint32_t kSH = 64;  // output rows per band
+constexpr uint32_t kMinRows = 4;
 
-hipError_t launch_fused(hipStream_t st, const LossViews& lv, const float4* img, const float4* target,
-                        float4* dl_out, double* partials, const CamParams* cams, const float2* tstats) {
-    const dim3 g(lv.block_begin[lv.n]);
-    if (g.x == 0) return hipSuccess;
-    if (tstats != nullptr)
-        hipLaunchKernelGGL((l1_ssim_fused_kernel<kSH, true>), g, dim3(256), 0, st, lv, img, target, dl_out,
-                           partials, cams, tstats);
-    else
-        hipLaunchKernelGGL((l1_ssim_fused_kernel<kSH, false>), g, dim3(256), 0, st, lv, img, target, dl_out,
-                           partials, cams, tstats);
+// Rows per band. A band of r rows works through r + 21 steps, the first 20 of
+// them short, so longer bands do less work; but the steps are serial, 1.1 us
+// each for a workgroup alone on its CU, and it takes four a CU to fill it
+// (1.95 us a step). Measured for c workgroups a CU (256 CUs): kStep[c] r +
+// kStart[c] us; more than four a CU run in rounds of four. The shortest
+// estimate is taken (a longer band where two agree). Against 64 rows always:
+// 256 x 256 89 -> 23 us, 1080p 104 -> 77 us, 1283 x 717 95 -> 52 us, eight
+// uneven views 382 -> 333 us, four 1080p 268 -> 249 us, sixteen 720p 483 ->
+// 428 us. dL/dimage does not depend on the bands; the double sums are grouped
+// by band, so a view's loss may differ in its last bits between launches.
+uint32_t band_rows(const LossViews& lv) {
+    constexpr float kStep[5] = {0.f, 1.1f, 1.3f, 1.65f, 1.95f}, kStart[5] = {0.f, 18.f, 22.f, 22.f, 22.f};
+    constexpr uint32_t kCus = 256;
+    uint32_t max_h = 0, best = kMinRows, strips[kMaxLossViews];
+    for (uint32_t j = 0; j < lv.n; ++j) {
+        max_h = std::max(max_h, lv.h[j]);
+        strips[j] = div_up(lv.w[j], kSW);
+    }
+    float best_us = INFINITY;
+    for (uint32_t r = kMinRows;; r += std::max(1u, r / 8)) {
+        const uint32_t bands = div_up(max_h, r), rows = std::max(kMinRows, div_up(max_h, bands));
+        uint64_t blocks = 0;
+        for (uint32_t j = 0; j < lv.n; ++j) blocks += (uint64_t)strips[j] * div_up(lv.h[j], rows);
+        const uint64_t rounds = blocks / (4 * kCus), c = div_up(blocks % (4 * kCus), (uint64_t)kCus);
+        const float us = (float)rounds * (kStep[4] * (float)rows + kStart[4]) + kStep[c] * (float)rows + kStart[c];
+        if (us <= best_us) {
+            best_us = us;
+            best = rows;
+        }
+        if (bands <= 1) return best;
+    }
+}
+
+hipError_t launch_fused(hipStream_t st, LossViews& lv, const float4* img, const float4* target, float4* dl_out,
+                        double* partials, const CamParams* cams, const float2* tstats) {
+    lv.rows = band_rows(lv);
+    uint32_t blocks = 0;
+    for (uint32_t j = 0; j < lv.n; ++j) {
+        lv.block_begin[j] = blocks;
+        blocks += div_up(lv.w[j], kSW) * div_up(lv.h[j], lv.rows);
+    }
+    lv.block_begin[lv.n] = blocks;
+    if (blocks == 0) return hipSuccess;
+    auto* kernel = tstats != nullptr ? l1_ssim_fused_kernel<true> : l1_ssim_fused_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, lv, img, target, dl_out, partials, cams, tstats);
     return hipGetLastError();
 }
 
@@ -392,7 +431,7 @@ void loss_weights(uint32_t w, uint32_t h, float lambda, float dssim_scale, float
 
 }  // namespace
 
-uint32_t l1_ssim_partials(uint32_t w, uint32_t h) { return div_up(w, kSW) * div_up(h, kSH); }
+uint32_t l1_ssim_partials(uint32_t w, uint32_t h) { return 1 + div_up(w, kSW) * div_up(h, kMinRows); }
 
 hipError_t launch_target_stats(hipStream_t st, uint32_t w, uint32_t h, const float4* target, float2* out) {
     const size_t P = (size_t)w * h;
@@ -412,7 +451,6 @@ hipError_t launch_l1_ssim(hipStream_t st, uint32_t w, uint32_t h, float lambda, 
     lv.w[0] = w;
     lv.h[0] = h;
     loss_weights(w, h, lambda, dssim_scale, &lv.dw[0], &lv.l1w[0]);
-    lv.block_begin[1] = l1_ssim_partials(w, h);
     return launch_fused(st, lv, img, target, dl_out, partial_sums, view, tstats);
 }
 
@@ -427,16 +465,12 @@ hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t first, uint32_t k, cons
     lv.n = k;
     lv.first = first;
     lv.partials_stride = partials_stride;
-    uint32_t blocks = 0;
     for (uint32_t j = 0; j < k; ++j) {
         lv.w[j] = widths[j];
         lv.h[j] = heights[j];
         lv.pix_base[j] = pix_base[j];
         loss_weights(widths[j], heights[j], lambda, dssim_scale, &lv.dw[j], &lv.l1w[j]);
-        lv.block_begin[j] = blocks;
-        blocks += l1_ssim_partials(widths[j], heights[j]);
     }
-    lv.block_begin[k] = blocks;
     return launch_fused(st, lv, img, target, dl_out, partials, cams_dev, tstats);
 }
 

@@ -206,7 +206,7 @@ constexpr uint32_t kSubWaves = AUX ? 5 : 6;
 // (FwdTrace; a verification variant, never used by training steps).
 template <bool AUX, int TW, int BATCH, bool TRACE = false>
 __global__ __launch_bounds__((TW / 8) * (TW / 8) * 64)
-__attribute__((amdgpu_waves_per_eu(kSubWaves<AUX>))) void raster_fwd_sub_kernel(
+__attribute__((amdgpu_waves_per_eu(TW == 8 ? 4 : kSubWaves<AUX>))) void raster_fwd_sub_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, FwdOut out, bool cull,
     uint32_t total_tiles, TileQueue queue, uint32_t tile_begin, FwdTrace trace) {

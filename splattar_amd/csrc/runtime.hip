@@ -1357,7 +1357,8 @@ static gs_status read_loss_partials(hipStream_t st, const double* partials, uint
     GS_HIP(hipStreamSynchronize(st));
     GS_HIP(hipMemcpy(p.data(), partials, p.size() * sizeof(double), hipMemcpyDeviceToHost));
     double l1 = 0.0, ss = 0.0;
-    for (uint32_t i = 0; i < n; ++i) {
+    n = std::min(n, 1u + (uint32_t)p[0]);
+    for (uint32_t i = 1; i < n; ++i) {
         l1 += p[2 * i];
         ss += p[2 * i + 1];
     }
