@@ -227,8 +227,7 @@ __global__ __launch_bounds__(256) void tile_order_keys_kernel(const uint32_t* __
     if (t < 2 * kTileQueues) cursors[t * kCursorStride] = 0u;
     if (t >= total_tiles) return;
     const size_t g = (size_t)tile_begin + t;
-    const uint32_t len = ranges[2 * g + 1] - ranges[2 * g];
-    keys[t] = 0xFFFFu - min(len, 0xFFFFu);
+    keys[t] = tile_order_key(ranges[2 * g + 1] - ranges[2 * g]);
     vals[t] = (uint32_t)g;
 }
 

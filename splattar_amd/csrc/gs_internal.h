@@ -649,6 +649,7 @@ hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_
 // keys[t] = 0xFFFF - min(list length, 0xFFFF), vals[t] = tile_begin + t,
 // *count = total_tiles and the 2 kTileQueues cursors = 0 (sort the pairs by
 // 16 key bits, stably, to get the order).
+__device__ __forceinline__ uint32_t tile_order_key(uint32_t len) { return 0xFFFFu - min(len, 0xFFFFu); }
 hipError_t launch_tile_order_keys(hipStream_t st, const uint32_t* ranges, uint32_t tile_begin,
                                   uint32_t total_tiles, uint32_t* keys, uint32_t* vals, uint32_t* count,
                                   uint32_t* cursors);
@@ -667,10 +668,18 @@ hipError_t launch_radix_sort_u64(hipStream_t st, uint64_t* keys0, uint32_t* vals
 hipError_t launch_copy_pairs(hipStream_t st, const void* src_keys, const uint32_t* src_vals,
                              void* dst_keys, uint32_t* dst_vals, uint32_t key_bytes,
                              const uint32_t* count, uint32_t capacity);
+// With `kept`, pairs whose key is kDropKey are left out and *kept receives the
+// number of the others.
+constexpr uint32_t kDropKey = 0xFFFFFFFFu;
 hipError_t launch_radix_sort_u32(hipStream_t st, uint32_t* keys0, uint32_t* vals0, uint32_t* keys1,
                                  uint32_t* vals1, const uint32_t* count, uint32_t capacity,
                                  uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
-                                 void* scratch, int* result_in_alt);
+                                 void* scratch, int* result_in_alt, uint32_t* kept = nullptr);
+// The order of launch_tile_order_keys, sorted, in one launch: up to
+// tile_order_small_cap() tiles.
+uint32_t tile_order_small_cap();
+hipError_t launch_tile_order_small(hipStream_t st, const uint32_t* ranges, uint32_t tile_begin, uint32_t n_tiles,
+                                   uint32_t* order, uint32_t* cursors);
 
 // raster_fwd.hip
 struct FwdOut {

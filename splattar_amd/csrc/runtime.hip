@@ -914,6 +914,11 @@ struct RasterCore {
         q_begin[slot] = t0;
         q_tiles[slot] = 0;
         if (!tile_queue || nt == 0) return GS_OK;
+        if (nt <= tile_order_small_cap()) {
+            GS_HIP(launch_tile_order_small(st, ranges, t0, nt, order_vals[0] + t0, cursors + 2 * slot * kCursorWords));
+            q_tiles[slot] = nt;
+            return GS_OK;
+        }
         GS_HIP(launch_tile_order_keys(st, ranges, t0, nt, order_keys[0] + t0, order_vals[0] + t0,
                                       order_count + slot, cursors + 2 * slot * kCursorWords));
         int alt = 0;
