@@ -280,16 +280,15 @@ __device__ __forceinline__ void pixel_s(const CamParams& cam, int x, int y, floa
 
 // One pixel-surfel evaluation (forward.rs:136-169), shared verbatim by the
 // forward and backward kernels so the backward replays the forward's alpha
-// decisions bit for bit. Returns alpha (0 when skipped).
+// decisions bit for bit.
 struct HitEval {
-    float alpha;     // min(o * ghat, 0.995), 0 if below 1/255
     float ghat;
     float u, v, t;   // ray-branch coordinates (t = centre depth on the screen branch)
     float inv_d;     // 1 / D (ray branch)
     float uv2;       // u^2 + v^2
     float raw;       // o * ghat
     float a;         // min(o * ghat, 0.995)
-    bool hit;        // a >= 1/255
+    bool hit;        // a >= 1/255; else the record is skipped
     bool ray;
     bool clamped;    // o * ghat > 0.995
 };
@@ -575,7 +574,6 @@ __device__ __forceinline__ HitEval eval_hit(const Record& r, float sx, float sy,
     h.clamped = h.raw > kAlphaClamp;
     h.a = fminf(h.raw, kAlphaClamp);
     h.hit = h.a >= kAlphaSkip;
-    h.alpha = h.hit ? h.a : 0.0f;
     return h;
 }
 

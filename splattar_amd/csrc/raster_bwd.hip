@@ -55,52 +55,85 @@ __device__ __forceinline__ float xlane(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xF, 0xF, false));
 }
 
-// One transposition step at lane bit OFF: lanes with the bit clear end up
-// with lo(self) + lo(partner), lanes with it set with hi(self) + hi(partner).
-// For OFF = 32 / 16 one v_permlane{32,16}_swap moves the upper half of lo
-// and the lower half of hi across in a single VALU op.
-template <int OFF>
-__device__ __forceinline__ float pair_sum(float lo, float hi, int lane) {
-    if constexpr (OFF == 32) {
-        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-        return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-    } else if constexpr (OFF == 16) {
-        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-        return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-    } else {
-        const bool upper = (lane & OFF) != 0;
-        const float send = upper ? lo : hi;
-        const float keep = upper ? hi : lo;
-        return keep + xlane<OFF>(send);
-    }
+// The largest x of the wave, as a scalar.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+    for (int o = 32; o >= 1; o >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, o));
+    return __builtin_amdgcn_readfirstlane(x);
 }
 
-template <int OFF>
-__device__ __forceinline__ float finish_sum(float r) {
-    if constexpr (OFF >= 1) return finish_sum<OFF / 2>(r + xlane<OFF>(r));
-    else return r;
+// Sums of values over the 64 lanes of a wave (every lane active) by halving: a
+// transposition step at lane bit OFF leaves lanes with the bit clear with
+// lo(self) + lo(partner) and lanes with it set with hi(self) + hi(partner), so
+// each step halves the values a lane holds; when one is left, the remaining
+// bits are summed. For bits 32 and 16 one permlane swap moves the upper half
+// of lo and the lower half of hi across. Within a 16-lane row the partner's
+// value comes by DPP (mirror, half mirror), and two adds that each write one
+// bank half replace two selects and an add. Written out because a swap through
+// the builtin copies an operand first: 16 values take 40 instructions instead
+// of 55, 6 % of the gradient pass at 1M surfels. s_nop 1: a swap or DPP reads
+// a register two waits after it is written.
+__device__ __forceinline__ void swap32(float (&a)[8], float (&b)[8]) {
+    asm("s_nop 1\n\t"
+        "v_permlane32_swap_b32 %0, %8\n\tv_permlane32_swap_b32 %1, %9\n\t"
+        "v_permlane32_swap_b32 %2, %10\n\tv_permlane32_swap_b32 %3, %11\n\t"
+        "v_permlane32_swap_b32 %4, %12\n\tv_permlane32_swap_b32 %5, %13\n\t"
+        "v_permlane32_swap_b32 %6, %14\n\tv_permlane32_swap_b32 %7, %15"
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
+          "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]), "+v"(b[6]), "+v"(b[7]));
 }
-
-template <int COUNT, int OFF, int NV>
-__device__ __forceinline__ float transpose_reduce(float (&v)[NV], int lane) {
-    if constexpr (COUNT > 1) {
+__device__ __forceinline__ void swap16(float (&a)[4], float (&b)[4]) {
+    asm("s_nop 1\n\t"
+        "v_permlane16_swap_b32 %0, %4\n\tv_permlane16_swap_b32 %1, %5\n\t"
+        "v_permlane16_swap_b32 %2, %6\n\tv_permlane16_swap_b32 %3, %7"
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+}
+// Lane l gets the total of value (l >> 2) & 15.
+__device__ __forceinline__ float wave_sums16(const float (&v)[16]) {
+    float a[8], b[8], c[4], d[4];
 #pragma unroll
-        for (int i = 0; i < COUNT / 2; ++i) v[i] = pair_sum<OFF>(v[i], v[COUNT / 2 + i], lane);
-        return transpose_reduce<COUNT / 2, OFF / 2, NV>(v, lane);
-    } else {
-        return finish_sum<OFF>(v[0]);
+    for (int i = 0; i < 8; ++i) {
+        a[i] = v[i];
+        b[i] = v[8 + i];
     }
+    swap32(a, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        c[i] = a[i] + b[i];
+        d[i] = a[4 + i] + b[4 + i];
+    }
+    swap16(c, d);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] += d[i];
+    float s, t;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %2, %2 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %1, %3, %3 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %0, %4, %4 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %5, %5 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+        "s_nop 1\n\t"
+        "v_add_f32_dpp %2, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %2, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "s_nop 1\n\t"
+        "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+        : "=&v"(s), "=&v"(t), "+v"(c[0])
+        : "v"(c[1]), "v"(c[2]), "v"(c[3]));
+    return c[0];
 }
-
-// Sum NV values (power of two, 4 <= NV <= 16) over the 64 lanes of a wave:
-// NV - 1 exchanges halve the value count per step, then the remaining lane
-// bits are summed. On return lane l holds the total of value index
-// (l >> log2(64/NV)) & (NV-1); lanes with (l & (64/NV - 1)) == 0 are the
-// designated writers.
-template <int NV>
-__device__ __forceinline__ float wave_reduce_transpose(float (&v)[NV], int lane) {
-    static_assert(NV >= 4 && NV <= 16 && (NV & (NV - 1)) == 0, "4, 8 or 16 values");
-    return transpose_reduce<NV, 32, NV>(v, lane);
+// Lane l gets the total of value (l >> 4) & 3.
+__device__ __forceinline__ float wave_sums4(const float (&v)[4]) {
+    auto swap = [](float lo, float hi, auto f) {
+        const auto p = f(__float_as_uint(lo), __float_as_uint(hi));
+        return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    };
+    auto s32 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+    auto s16 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+    float r = swap(swap(v[0], v[2], s32), swap(v[1], v[3], s32), s16);
+    r += xlane<8>(r);
+    r += xlane<4>(r);
+    r += xlane<2>(r);
+    return r + xlane<1>(r);
 }
 
 // Per-pixel state of the backward walk.
@@ -177,7 +210,7 @@ __device__ __forceinline__ void step_aux_sums(PixState& p, const Record& r, floa
 // does to T and the suffix sums.
 template <bool AUX>
 __device__ __forceinline__ void step_state(PixState& p, const Record& r, const HitEval& h, bool act, float lambda) {
-    const float alpha = act ? h.alpha : 0.0f;
+    const float alpha = act ? h.a : 0.0f;
     const float t_before = p.T * rcp_refined(1.0f - alpha);
     const float w = t_before * alpha;
     p.suf_r = fmaf(r.col_op.x, w, p.suf_r);
@@ -265,7 +298,7 @@ __device__ __forceinline__ void put(float& dst, float v) {
 template <bool AUX, bool ACC>
 __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitEval& h, bool act,
                                         float lambda, float (&g)[16], float (&g2)[4]) {
-    const float alpha = act ? h.alpha : 0.0f;
+    const float alpha = act ? h.a : 0.0f;
     const float inv_one_m = rcp_refined(1.0f - alpha);
     const float t_before = p.T * inv_one_m;
     const float w = t_before * alpha;
@@ -397,8 +430,8 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
         load_pixel<AUX>(pa, cam, px, py, in, lambda);
         if constexpr (TWO) load_pixel<AUX>(pb, cam, px, py + 8, in, lambda);
         else pb.last = 0u;
-        const uint32_t mylast = max(pa.last, pb.last);
-        if (mylast) atomicMax(&s_maxlast, mylast);
+        const uint32_t last_a = wave_max(pa.last), last_b = wave_max(pb.last);
+        if (lane == 0) atomicMax(&s_maxlast, max(last_a, last_b));
         __syncthreads();
         const uint32_t maxlast = s_maxlast;
         if (maxlast == 0) continue;
@@ -485,8 +518,8 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 const uint32_t rel = first + j;
                 // A block is walked only while some pixel of it is at or before
                 // its last contributor (a pixel past it changes nothing).
-                const bool need_a = top && __any(rel < pa.last);
-                const bool need_b = bot && __any(rel < pb.last);
+                const bool need_a = top && rel < last_a;
+                const bool need_b = bot && rel < last_b;
                 if (!need_a && !need_b) continue;
                 Record r;
                 r.m_nt = s_m[j];
@@ -501,11 +534,11 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 bool act_a = false, act_b = false;
                 if (need_a) {
                     ha = eval_hit(r, pa.sx, pa.sy, pa.pxc, pa.pyc);
-                    act_a = rel < pa.last && ha.alpha > 0.0f;
+                    act_a = rel < pa.last && ha.hit;
                 }
                 if (need_b) {
                     hb = eval_hit(r, pb.sx, pb.sy, pb.pxc, pb.pyc);
-                    act_b = rel < pb.last && hb.alpha > 0.0f;
+                    act_b = rel < pb.last && hb.hit;
                 }
                 const bool go_a = need_a && __any(act_a);
                 const bool go_b = need_b && __any(act_b);
@@ -523,7 +556,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 } else {
                     add_hit<AUX, false>(pb, r, hb, act_b, lambda, g, g2);
                 }
-                const float red = wave_reduce_transpose<16>(g, lane);
+                const float red = wave_sums16(g);
                 if ((lane & 3) == 0) {
                     float* const dst = &s_grad[NG > 1 ? wave : 0][j * NS + (lane >> 2)];
                     if constexpr (NG == NW) *dst = red;
@@ -531,7 +564,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 }
                 if (AUX) {
                     static_assert(!AUX || NG == NW, "a copy of the slots per wave");
-                    const float red2 = wave_reduce_transpose<4>(g2, lane);
+                    const float red2 = wave_sums4(g2);
                     if ((lane & 15) == 0) s_grad[NG > 1 ? wave : 0][j * NS + 16 + (lane >> 4)] = red2;
                 }
             }
@@ -572,12 +605,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
     BwdSegments sg) {
     constexpr int NS = grad_stride(false);
     constexpr int SPT = BATCH / 64;          // staging rounds per batch
-    constexpr int MB = 10;                   // list entry: slot | block mask << MB
-    static_assert(BATCH % 64 == 0 && BATCH <= (1 << MB), "batch of whole waves");
+    // List entry: slot | block mask << 8 | channels at 0 (bits 12, 16, 20).
+    static_assert(BATCH % 64 == 0 && BATCH <= 256, "batch of whole waves");
     __shared__ float4 s_m[BATCH], s_a[BATCH], s_b[BATCH], s_c[BATCH];
     __shared__ uint32_t s_pay[BATCH];
-    __shared__ uint16_t s_list[BATCH];
+    __shared__ uint32_t s_list[BATCH + 1];  // read one entry ahead
 
+    constexpr uint64_t kWriters = 0x1111111111111111ull;  // lane 4 k holds total k
     const int lane = threadIdx.x;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const uint32_t nseg = sg.state != nullptr ? min(sg.ctl[0], sg.pool) : 0u;
@@ -603,15 +637,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
         const uint32_t tx = local % cam.tiles_x, ty = local / cam.tiles_x;
         const uint32_t x0 = tx * 16, y0 = ty * 16;
         PixState p[4];
-        uint32_t mylast = 0;
+        uint32_t block_last[4], maxlast = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             load_pixel<false>(p[q], cam, (int)x0 + 8 * (q & 1) + (lane & 7), (int)y0 + 8 * (q >> 1) + (lane >> 3),
                               in, 0.0f);
-            mylast = max(mylast, p[q].last);
+            block_last[q] = wave_max(p[q].last);
+            maxlast = max(maxlast, block_last[q]);
         }
-        for (int o = 32; o >= 1; o >>= 1) mylast = max(mylast, (uint32_t)__shfl_xor((int)mylast, o));
-        const uint32_t maxlast = __builtin_amdgcn_readfirstlane(mylast);
         if (maxlast == 0) continue;
         // The list positions [k0, k1) of this item.
         uint32_t k0 = 0, k1 = maxlast;
@@ -634,7 +667,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
 #pragma unroll
             for (int m = 0; m < SPT; ++m) {
                 const int slot = lane + m * 64;
-                uint32_t qmask = 0;
+                uint32_t qmask = 0, dark = 0;
                 if ((uint32_t)slot < cnt) {
                     const uint32_t pay = payloads[base + slot];
                     Record r = recs[pay];
@@ -644,27 +677,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                     s_b[slot] = r.b_py;
                     s_c[slot] = r.col_op;
                     qmask = cull ? block_mask<16>(r, x0, y0) : 0xFu;
+                    // A block is walked only from its last contributor on.
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (first_k + (uint32_t)slot >= block_last[q]) qmask &= ~(1u << q);
+                    // A colour channel clamped at 0 in the forward passes no
+                    // gradient to SH (the record stores it as exactly 0).
+                    dark = (r.col_op.x == 0.0f ? 1u : 0u) | (r.col_op.y == 0.0f ? 0x10u : 0u) |
+                           (r.col_op.z == 0.0f ? 0x100u : 0u);
                 }
                 const uint64_t bal = __ballot(qmask != 0u);
                 if (qmask != 0u)
-                    s_list[count + (uint32_t)__popcll(bal & lt_mask)] = (uint16_t)(slot | (qmask << MB));
+                    s_list[1 + count + (uint32_t)__popcll(bal & lt_mask)] = (uint32_t)slot | (qmask << 8) | (dark << 12);
                 count += (uint32_t)__popcll(bal);
             }
             __syncthreads();
 
-            for (int kk = (int)count - 1; kk >= 0; --kk) {
-                const uint32_t e = __builtin_amdgcn_readfirstlane((uint32_t)s_list[kk]);
-                const uint32_t j = e & ((1u << MB) - 1u);
-                const uint32_t qm = e >> MB;
+            uint32_t next = s_list[count];
+            for (uint32_t kk = count; kk > 0; --kk) {
+                const uint32_t e = __builtin_amdgcn_readfirstlane(next);
+                next = s_list[kk - 1];
+                const uint32_t j = e & 0xFFu;
                 const uint32_t rel = first_k + j;
-                bool need[4];
-                bool any_need = false;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    need[q] = ((qm >> q) & 1u) && __any(rel < p[q].last);
-                    any_need = any_need || need[q];
-                }
-                if (!any_need) continue;
                 Record r;
                 r.m_nt = s_m[j];
                 r.a_px = s_a[j];
@@ -673,31 +707,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                 r.nrm_dep = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 float g[16];
                 float g2[4];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) asm volatile("" : "=v"(g[k]));  // defined here: else copied before the sums
                 g[kGNt] = 0.0f;
-                bool first = true;
+                uint32_t blocks = 0;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    if (!need[q]) continue;
+                    if (((e >> (8 + q)) & 1u) == 0u) continue;
                     const HitEval h = eval_hit(r, p[q].sx, p[q].sy, p[q].pxc, p[q].pyc);
-                    const bool act = rel < p[q].last && h.alpha > 0.0f;
+                    const bool act = rel < p[q].last && h.hit;
                     if (!__any(act)) continue;
-                    if (first) add_hit<false, false>(p[q], r, h, act, 0.0f, g, g2);
+                    if (blocks == 0u) add_hit<false, false>(p[q], r, h, act, 0.0f, g, g2);
                     else add_hit<false, true>(p[q], r, h, act, 0.0f, g, g2);
-                    first = false;
+                    blocks = 1u;
                 }
-                if (first) continue;
-                const float red = wave_reduce_transpose<16>(g, lane);
-                if ((lane & 3) == 0 && red != 0.0f) {
-                    const int slot = lane >> 2;
-                    bool keep = true;
-                    if (slot >= kGCol && slot < kGCol + 3) {
-                        // A colour channel clamped at 0 in the forward passes no
-                        // gradient to SH (the record stores it as exactly 0).
-                        const float4 c = s_c[j];
-                        keep = (slot == kGCol ? c.x : (slot == kGCol + 1 ? c.y : c.z)) != 0.0f;
-                    }
-                    if (keep) atomicAdd(&grad_coef[(size_t)s_pay[j] * NS + slot], red);
-                }
+                if (blocks == 0u) continue;
+                const float red = wave_sums16(g);
+                const uint64_t writers = kWriters & ~((uint64_t)(e >> 12) << (4 * kGCol));
+                float* const dst = grad_coef + (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(s_pay[j]) * NS;
+                if (__builtin_amdgcn_inverse_ballot_w64(writers) && red != 0.0f) atomicAdd(dst + (lane >> 2), red);
             }
         }
     }
@@ -832,7 +860,7 @@ __global__ __launch_bounds__(256) void raster_state_kernel(
                     r.col_op = s_rec[3][j];
                     r.nrm_dep = AUX ? s_n[AUX ? j : 0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                     const HitEval h = eval_hit(r, ps.sx, ps.sy, ps.pxc, ps.pyc);
-                    step_state<AUX>(ps, r, h, first + j < ps.last && h.alpha > 0.0f, lambda);
+                    step_state<AUX>(ps, r, h, first + j < ps.last && h.hit, lambda);
                 }
             }
             store_state<AUX>(sg, at + s - 1, pixel, ps);

@@ -143,13 +143,13 @@ __global__ __launch_bounds__((TW / 8) * (TW / 8) * 64) void raster_fwd_kernel(
                 };
                 auto composite = [&](uint32_t j, const Record& r) {
                     const HitEval h = eval_hit(r, sx, sy, pxc, pyc);
-                    if (T >= kTTerminate && h.alpha > 0.0f) {
-                        const float w = T * h.alpha;
+                    if (T >= kTTerminate && h.hit) {
+                        const float w = T * h.a;
                         cr += r.col_op.x * w;
                         cg += r.col_op.y * w;
                         cb += r.col_op.z * w;
                         wsum += w;
-                        T *= 1.0f - h.alpha;
+                        T *= 1.0f - h.a;
                         last = base - start + j + 1u;
                     }
                 };
@@ -319,7 +319,7 @@ __attribute__((amdgpu_waves_per_eu(TW == 8 ? 4 : kSubWaves<AUX>))) void raster_f
                 const uint32_t first = base - start + 1;
                 auto composite = [&](uint32_t j, const Record& r, bool listed) {
                     const HitEval h = eval_hit(r, sx, sy, pxc, pyc);
-                    if (listed && T >= kTTerminate && h.hit) {
+                    if (listed & (T >= kTTerminate) & h.hit) {
                         const float w = T * h.a;
                         cr += r.col_op.x * w;
                         cg += r.col_op.y * w;
