@@ -324,8 +324,10 @@ __device__ inline void record_footprint(Record& r, const CamParams& cam) {
         r.ell1 = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
         return;
     }
-    const double L = log((double)op * 255.0) + 2e-3;
-    const double rs = sqrt(L) + kMargin;
+    // Logarithm and roots of it in f32 (1e-6, well inside the 2e-3), one f64
+    // division for all quotients by det2: half of the f64 instructions.
+    const double L = (double)__logf(op * 255.0f) + 2e-3;
+    const double rs = (double)(sqrtf((float)L) + kMargin);
     double x0 = r.a_px.w - rs, x1 = r.a_px.w + rs, y0 = r.b_py.w - rs, y1 = r.b_py.w + rs;
     const double k = 2.0 * L;
     const double A[3] = {r.a_px.x, r.a_px.y, r.a_px.z};
@@ -364,6 +366,7 @@ __device__ inline void record_footprint(Record& r, const CamParams& cam) {
     bool bounded = Q[0][0] > 0.0 && det2 > 1e-5 * mag;
     double ex = kFar, ey = kFar, h00 = 1.0, h01 = 0.0, h11 = 1.0;  // empty ellipse by default
     if (bounded) {
+        const double id = 1.0 / det2;
         const double a00 = Q[1][1] * Q[2][2] - Q[1][2] * Q[1][2];
         const double a11 = Q[0][0] * Q[2][2] - Q[0][2] * Q[0][2];
         const double a02 = Q[0][1] * Q[1][2] - Q[0][2] * Q[1][1];
@@ -372,19 +375,19 @@ __device__ inline void record_footprint(Record& r, const CamParams& cam) {
         bounded = dx >= 0.0 && dy >= 0.0;
         if (bounded) {
             const double sdx = sqrt(dx), sdy = sqrt(dy);
-            const double sx_lo = (a02 - sdx) / det2, sx_hi = (a02 + sdx) / det2;
-            const double sy_lo = (a12 - sdy) / det2, sy_hi = (a12 + sdy) / det2;
+            const double sx_lo = (a02 - sdx) * id, sx_hi = (a02 + sdx) * id;
+            const double sy_lo = (a12 - sdy) * id, sy_hi = (a12 + sdy) * id;
             // X = cx - f sx (pixel centre), Y = cy + f sy.
             x0 = fmin(x0, cam.cx - f * sx_hi - kMargin);
             x1 = fmax(x1, cam.cx - f * sx_lo + kMargin);
             y0 = fmin(y0, cam.cy + f * sy_lo - kMargin);
             y1 = fmax(y1, cam.cy + f * sy_hi + kMargin);
         }
-        const double csx = -(Q[1][1] * Q[0][2] - Q[0][1] * Q[1][2]) / det2;
-        const double csy = -(Q[0][0] * Q[1][2] - Q[0][1] * Q[0][2]) / det2;
+        const double csx = -(Q[1][1] * Q[0][2] - Q[0][1] * Q[1][2]) * id;
+        const double csy = -(Q[0][0] * Q[1][2] - Q[0][1] * Q[0][2]) * id;
         const double qc = Q[2][2] + Q[0][2] * csx + Q[1][2] * csy;
         if (bounded && qc < 0.0) {
-            const double sc = 1.0 / (-qc * f * f * (1.0 + 2e-6 * Q[0][0] * Q[1][1] / det2));
+            const double sc = 1.0 / (-qc * f * f * (1.0 + 2e-6 * Q[0][0] * Q[1][1] * id));
             ex = cam.cx - f * csx;
             ey = cam.cy + f * csy;
             h00 = Q[0][0] * sc;
@@ -402,7 +405,7 @@ __device__ inline void record_footprint(Record& r, const CamParams& cam) {
     }
     r.box = make_float4((float)x0, (float)y0, (float)x1, (float)y1);
     r.ell0 = make_float4((float)ex, (float)ey, (float)h00, (float)h01);
-    r.ell1 = make_float4((float)h11, (float)(1.0 / h00), (float)(1.0 / h11), (float)rs);
+    r.ell1 = make_float4((float)h11, 1.0f / (float)h00, 1.0f / (float)h11, (float)rs);
 }
 
 // True when the record's footprint can reach the pixel-centre rectangle
@@ -448,16 +451,16 @@ __device__ __forceinline__ uint32_t block_mask(const Record& r, uint32_t x0, uin
     return m;
 }
 
-// Footprint against the 4x4 sub-blocks of a tile, one row of sub-blocks at a
-// time: the ellipse's and the disk's x extents over the row's y range give a
-// column interval, cut by the box. In offsets from the centre the ellipse is
+// Footprint against a row of equal blocks (the 4x4 sub-blocks of a tile, the
+// tiles of a rect): the ellipse's and the disk's x extents over the row's y
+// range give a column interval. In offsets from the centre the ellipse is
 // x = -k y -+ sqrt(i00 - q y^2), k = h01 / h00, q = det / h00^2; over a y
 // interval its right edge is concave with its maximum at y = -ys (the
 // ellipse's own extreme) and its left edge convex with its minimum at ys, so
 // each is evaluated at that y clamped to the interval. kSubMargin px of margin
 // (in f32, ys of a thin diagonal ellipse is off by 1e-7 kappa, which costs its
 // tip up to 0.03 of the short axis on top of footprint_hits' errors), and the
-// hull of the two extents: never fewer sub-blocks than the record reaches.
+// hull of the two extents: never fewer blocks than the record reaches.
 constexpr float kSubMargin = 0.125f;
 struct SubTest {
     float4 box;
@@ -480,29 +483,34 @@ __device__ __forceinline__ SubTest sub_test(float4 box, float4 e0, float4 e1, fl
     t.ys = e0.w * e1.z * __builtin_amdgcn_sqrtf(e1.x * __builtin_amdgcn_rcpf(det));
     return t;
 }
+// The x extent [xl, xr] of the footprint over the pixel centres ylo .. yhi,
+// without the margin in x; xl > xr when it does not reach them.
+__device__ __forceinline__ void row_extent(const SubTest& t, float ylo, float yhi, float& xl, float& xr) {
+    if (t.i00 == 0.0f) {
+        xl = -kFar;
+        xr = kFar;
+        return;
+    }
+    const float da = ylo - kSubMargin - t.ey, db = yhi + kSubMargin - t.ey;
+    const float yr = fminf(fmaxf(-t.ys, da), db), yl = fminf(fmaxf(t.ys, da), db);
+    const float dr = fmaf(-t.q * yr, yr, t.i00), dl = fmaf(-t.q * yl, yl, t.i00);
+    // The strip meets the ellipse in both or in neither (rounding aside).
+    const float slack = -1e-3f * t.i00;
+    const bool hit = dr >= slack || dl >= slack;
+    xr = hit ? t.ex - t.k * yr + __builtin_amdgcn_sqrtf(fmaxf(dr, 0.0f)) : -kFar;
+    xl = hit ? t.ex - t.k * yl - __builtin_amdgcn_sqrtf(fmaxf(dl, 0.0f)) : kFar;
+    const float dy = fminf(fmaxf(t.py, ylo - kSubMargin), yhi + kSubMargin) - t.py;
+    const float h2 = fmaf(-dy, dy, t.rd2);
+    const float hx = __builtin_amdgcn_sqrtf(fmaxf(h2, 0.0f));
+    xr = h2 >= 0.0f ? fmaxf(xr, t.px + hx) : xr;
+    xl = h2 >= 0.0f ? fminf(xl, t.px - hx) : xl;
+}
 // Bit c: the record's footprint can reach the sub-block of pixel centres
 // [x0 + 4 c + 0.5, + 3] x [y0 + 0.5, + 3].
 __device__ __forceinline__ uint32_t sub_row_mask(const SubTest& t, float x0, float y0) {
     const float ylo = y0 + 0.5f, yhi = y0 + 3.5f;
     float xl, xr;
-    if (t.i00 == 0.0f) {
-        xl = -kFar;
-        xr = kFar;
-    } else {
-        const float da = ylo - kSubMargin - t.ey, db = yhi + kSubMargin - t.ey;
-        const float yr = fminf(fmaxf(-t.ys, da), db), yl = fminf(fmaxf(t.ys, da), db);
-        const float dr = fmaf(-t.q * yr, yr, t.i00), dl = fmaf(-t.q * yl, yl, t.i00);
-        // The strip meets the ellipse in both or in neither (rounding aside).
-        const float slack = -1e-3f * t.i00;
-        const bool hit = dr >= slack || dl >= slack;
-        xr = hit ? t.ex - t.k * yr + __builtin_amdgcn_sqrtf(fmaxf(dr, 0.0f)) : -kFar;
-        xl = hit ? t.ex - t.k * yl - __builtin_amdgcn_sqrtf(fmaxf(dl, 0.0f)) : kFar;
-        const float dy = fminf(fmaxf(t.py, ylo - kSubMargin), yhi + kSubMargin) - t.py;
-        const float h2 = fmaf(-dy, dy, t.rd2);
-        const float hx = __builtin_amdgcn_sqrtf(fmaxf(h2, 0.0f));
-        xr = h2 >= 0.0f ? fmaxf(xr, t.px + hx) : xr;
-        xl = h2 >= 0.0f ? fminf(xl, t.px - hx) : xl;
-    }
+    row_extent(t, ylo, yhi, xl, xr);
     // Columns [lo, hi]: x0 + 4 c + 3.5 >= left edge, x0 + 4 c + 0.5 <= right edge.
     const float lo = fmaxf(xl - (3.5f + kSubMargin), t.box.x - 3.5f) - x0;
     const float hi = fminf(xr - (0.5f - kSubMargin), t.box.z - 0.5f) - x0;
@@ -511,6 +519,17 @@ __device__ __forceinline__ uint32_t sub_row_mask(const SubTest& t, float x0, flo
     const uint32_t m = ((1u << (ch + 1)) - 1u) & ~((1u << cl) - 1u);
     const bool rows = t.box.w >= ylo && t.box.y <= yhi && ch >= 0;
     return rows ? m : 0u;
+}
+// Bits of the tiles (size ts px) x0 .. x0 + w - 1 of tile row y that the
+// footprint can reach (1 <= w <= 64).
+__device__ __forceinline__ uint64_t tile_row_mask(const SubTest& t, uint32_t x0, uint32_t w, uint32_t y, uint32_t ts) {
+    const float span = (float)ts - 0.5f, first = (float)(x0 * ts), top = (float)(y * ts);
+    float xl, xr;
+    row_extent(t, top + 0.5f, top + span, xl, xr);
+    const float inv = 1.0f / (float)ts;
+    const int cl = (int)ceilf(fminf(fmaxf((xl - (span + kSubMargin) - first) * inv, 0.0f), 64.0f));
+    const int ch = (int)floorf(fminf(fmaxf((xr - (0.5f - kSubMargin) - first) * inv, -1.0f), (float)(w - 1u)));
+    return ch < cl ? 0ull : (~0ull >> (63 - (ch - cl))) << cl;
 }
 
 // Cuts a footprint box (pixel centres) to the pixels of the kTile rect
@@ -598,8 +617,7 @@ inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) /
 // project.hip
 // presort_keys / presort_vals (optional) receive a copy of the depth key and
 // the item index for the depth presort; item_count (optional) receives
-// n * n_views; rects / depth_keys / counts may be null; write_normal false
-// leaves Record::nrm_dep unwritten (colour-only consumers).
+// n * n_views; rects / depth_keys / counts may be null.
 hipError_t launch_project(hipStream_t st, const CamParams* cams_dev, uint32_t n_views, uint32_t n,
                           const float4* pos, const float2* scales, const float4* quats,
                           const float* opac, const float* sh, Record* recs, uint4* rects,
@@ -607,7 +625,7 @@ hipError_t launch_project(hipStream_t st, const CamParams* cams_dev, uint32_t n_
                           uint32_t num_ranges, uint32_t* presort_keys = nullptr,
                           uint32_t* presort_vals = nullptr, uint32_t* item_count = nullptr,
                           bool clip_to_box = false, uint4* emit_info = nullptr,
-                          bool pack_counts = false, bool write_normal = true);
+                          bool pack_counts = false);
 
 // scan.hip
 // Items per scan partition; the scratch holds a 256-B header and one u32 sum

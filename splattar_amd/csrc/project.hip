@@ -12,8 +12,7 @@
 // binning); without it, the 16-px rect itself (work tiles must be 16 px).
 // Surfels i >= cam.n_surfels are culled in that view. rects, depth_keys and
 // counts may be null (callers that read only the presort and emit_info
-// outputs); with write_normal false the record's normal / depth float4 is
-// not written (colour-only consumers never read it).
+// outputs).
 
 #include "gs_internal.h"
 
@@ -28,7 +27,7 @@ __global__ __launch_bounds__(256) void project_kernel(
     uint4* __restrict__ rects, uint32_t* __restrict__ depth_keys, uint32_t* __restrict__ counts,
     uint32_t* __restrict__ ranges_to_clear, uint32_t num_ranges, uint32_t* __restrict__ presort_keys,
     uint32_t* __restrict__ presort_vals, uint32_t* __restrict__ item_count, bool clip_to_box,
-    uint4* __restrict__ emit_info, bool pack_counts, bool write_normal) {
+    uint4* __restrict__ emit_info, bool pack_counts) {
     // Views vary fastest over the logical blocks and each XCD takes a
     // contiguous range of them, so the V blocks that read the same 256
     // surfels run on one XCD and the later ones find the parameters in its L2.
@@ -43,8 +42,8 @@ __global__ __launch_bounds__(256) void project_kernel(
         for (uint32_t k = i; k < num_ranges; k += sblocks * blockDim.x) ranges_to_clear[k] = 0u;
     }
     if (view == 0 && i == 0 && item_count != nullptr) *item_count = n * n_views;
-    // Every thread of the block runs to the cooperative tile-mask step below
-    // (it uses the whole wave); items past n only take part with no tiles.
+    // Every thread of the block runs to the store of the records below; items
+    // past n have none.
     const bool in_range = i < n;
     const CamParams cam = cams[view];
     const uint32_t g = view * n + i;
@@ -111,90 +110,21 @@ __global__ __launch_bounds__(256) void project_kernel(
         }
     }
 
-    // Per-tile footprint masks, wave-cooperatively: the (item, tile) pairs of
-    // the wave's masked items are dealt 64 at a time over the lanes (owner by
-    // binary search over the wave's exclusive scan of tile counts), each lane
-    // tests one tile against its owner's footprint read from LDS; an owner's
-    // pairs of a round are consecutive lanes, so its bits are a shifted slice
-    // of the round's ballot, merged into its mask by the run's first lane.
-    // Bit t = row-major tile t of the rect.
-    // The cost follows the wave's total tile count, not 64 x its widest item.
-    // s_stage holds the footprints for the masks (s_fp), then the block's
-    // records for one contiguous store (rows of kRecRow float4, one spare
-    // against LDS bank conflicts).
-    constexpr int kRecRow = 9;
-    __shared__ float4 s_stage[256 * kRecRow];
-    __shared__ uint32_t s_bits[256][2];
-    __shared__ uint32_t s_write[256];
-    // Field-major (lane-consecutive 16-B accesses): box, ell0, ell1, (px, py, rect width, 0).
-    float4 (*s_fp)[256] = reinterpret_cast<float4 (*)[256]>(s_stage);
-    {
-        const int tid = threadIdx.x, lane = tid & 63, wbase = tid & ~63;
-        const uint32_t mine = masked ? count : 0u;
-        const uint32_t rw = rect.z - rect.x + 1u;
-        if (masked) {
-            s_fp[0][tid] = rec.box;
-            s_fp[1][tid] = rec.ell0;
-            s_fp[2][tid] = rec.ell1;
-            s_fp[3][tid] = make_float4(rec.a_px.w, rec.b_py.w, (float)rw, 0.0f);
-        }
-        s_bits[tid][0] = 0u;
-        s_bits[tid][1] = 0u;
-        uint32_t incl = mine;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t v = __shfl_up(incl, o);
-            if (lane >= o) incl += v;
-        }
-        const uint32_t total = __shfl(incl, 63);
-        const uint32_t excl = incl - mine;
-        __syncthreads();
-        const uint32_t ts = cam.tile_size;
-        const float span = (float)ts - 0.5f;
-        for (uint32_t k0 = 0; k0 < total; k0 += 64) {
-            const uint32_t k = k0 + (uint32_t)lane;
-            int owner = 0;
-            for (int step = 32; step >= 1; step >>= 1) {
-                const int cand = owner + step;
-                const uint32_t ex = __shfl(excl, cand & 63);
-                if (cand < 64 && ex <= k) owner = cand;
-            }
-            const uint32_t o_excl = __shfl(excl, owner);
-            const uint32_t o_end = o_excl + __shfl(mine, owner);
-            const uint32_t o_x0 = __shfl(rect.x, owner), o_y0 = __shfl(rect.y, owner);
-            const int prev_owner = __shfl_up(owner, 1);
-            const uint32_t t = k - o_excl;
-            bool hit = false;
-            if (k < total) {
-                const float4 q3 = s_fp[3][wbase + owner];
-                const uint32_t w = (uint32_t)q3.z;
-                // t < 64 and w <= 64: the float quotient's floor is exact.
-                const uint32_t ty = (uint32_t)(((float)t + 0.5f) / q3.z);
-                const uint32_t tx = t - ty * w;
-                Record fr;
-                fr.box = s_fp[0][wbase + owner];
-                fr.ell0 = s_fp[1][wbase + owner];
-                fr.ell1 = s_fp[2][wbase + owner];
-                fr.a_px.w = q3.x;
-                fr.b_py.w = q3.y;
-                const float px0 = (float)((o_x0 + tx) * ts), py0 = (float)((o_y0 + ty) * ts);
-                hit = footprint_hits(fr, px0 + 0.5f, py0 + 0.5f, px0 + span, py0 + span);
-            }
-            const uint64_t bal = __ballot(hit);
-            if (k < total && (lane == 0 || prev_owner != owner)) {
-                // This lane starts its owner's run of the round: lanes
-                // [lane, lane + run) hold tiles t .. t + run - 1 (t + run <= 64).
-                const uint32_t run = min(o_end, k0 + 64u) - k;
-                const uint64_t seg = run >= 64u ? ~0ull : ((1ull << run) - 1ull);
-                const uint64_t bits = ((bal >> lane) & seg) << t;
-                s_bits[wbase + owner][0] |= (uint32_t)bits;
-                s_bits[wbase + owner][1] |= (uint32_t)(bits >> 32);
-            }
-        }
-        __syncthreads();
-        if (masked) {
-            mask = (uint64_t)s_bits[tid][0] | ((uint64_t)s_bits[tid][1] << 32);
-            count = (uint32_t)__popcll(mask);
-        }
+    // Per-tile footprint masks, bit t = row-major tile t of the rect: each lane
+    // takes the rows of its item's rect, a column interval for each (a rect is
+    // a few tiles; the wave takes as many steps as its tallest rect has rows).
+    // Dealing (item, tile) pairs over the lanes, with an owner search and a
+    // footprint test a pair, took half of the kernel's LDS accesses and a
+    // quarter of its instructions. In all 367 -> 274 us for 4M items and 1200 ->
+    // 983 us for 20M (where 128 B a record written and the parameters read take
+    // 0.15 and 0.6 ms).
+    if (masked) {
+        const SubTest t = sub_test(rec.box, rec.ell0, rec.ell1, rec.a_px.w, rec.b_py.w);
+        const uint32_t w = rect.z - rect.x + 1u;
+        mask = 0ull;
+        for (uint32_t y = rect.y, shift = 0u; y <= rect.w; ++y, shift += w)
+            mask |= tile_row_mask(t, rect.x, w, y, cam.tile_size) << shift;
+        count = (uint32_t)__popcll(mask);
     }
     // Binning outputs; a record only for items that reach a tile (no entry
     // ever reads the others).
@@ -217,7 +147,9 @@ __global__ __launch_bounds__(256) void project_kernel(
         float basis[16];
         const int nb = sh_basis((int)cam.sh_degree, f.xx * inv_len, f.xy * inv_len, f.xz * inv_len, basis);
         // 16-B loads of the (48-float, 192-B aligned) coefficient row, only as
-        // far as the degree needs.
+        // far as the degree needs; all at once: four at a time (80 registers
+        // and six waves a SIMD instead of 103 and four) take 314 instead of
+        // 274 us for 4M items.
         const float4* sh4 = reinterpret_cast<const float4*>(sh + (size_t)i * kShFloats);
         float shv[kShFloats];
 #pragma unroll
@@ -249,29 +181,39 @@ __global__ __launch_bounds__(256) void project_kernel(
         rec.nrm_dep = make_float4(nrm.x, nrm.y, nrm.z, depth);
     }
     // The block's items are consecutive (one view, 256 consecutive surfels):
-    // stage the records in LDS and store them as one run, lane-consecutive
-    // 16-B stores instead of eight 16-B stores at a 128-B stride per lane.
-    {
-        const int tid = threadIdx.x;
-        s_write[tid] = write_rec ? 1u : 0u;
-        if (write_rec) {
-            float4* row = s_stage + tid * kRecRow;
-            row[0] = rec.m_nt;
-            row[1] = rec.a_px;
-            row[2] = rec.b_py;
-            row[3] = rec.col_op;
-            row[4] = rec.nrm_dep;
-            row[5] = rec.box;
-            row[6] = rec.ell0;
-            row[7] = rec.ell1;
+    // stage the records in LDS, half the block at a time, and store them as one
+    // run, lane-consecutive 16-B stores instead of eight 16-B stores at a
+    // 128-B stride per lane. Whole 128-B records, the normal also where nothing
+    // reads it: a record with a 16-B hole costs a read of its line (4M records
+    // 377 us against 310, 20M 1150 against 1020).
+    constexpr int kRecRow = 9;  // float4 a row: one spare against LDS bank conflicts
+    __shared__ float4 s_stage[128 * kRecRow];
+    __shared__ uint32_t s_write[128];
+    const uint32_t tid = threadIdx.x, i0 = i - tid;
+    const uint32_t nrec = i0 < n ? min(256u, n - i0) : 0u;
+#pragma unroll
+    for (uint32_t half = 0; half < 2; ++half) {
+        if (half == 1) __syncthreads();  // the first half's rows are stored
+        if (tid >> 7 == half) {
+            s_write[tid & 127u] = write_rec ? 1u : 0u;
+            if (write_rec) {
+                float4* row = s_stage + (tid & 127u) * kRecRow;
+                row[0] = rec.m_nt;
+                row[1] = rec.a_px;
+                row[2] = rec.b_py;
+                row[3] = rec.col_op;
+                row[4] = rec.nrm_dep;
+                row[5] = rec.box;
+                row[6] = rec.ell0;
+                row[7] = rec.ell1;
+            }
         }
         __syncthreads();
-        const uint32_t i0 = i - (uint32_t)tid;
-        const uint32_t nrec = i0 < n ? min(256u, n - i0) : 0u;
-        float4* dst = reinterpret_cast<float4*>(recs + (size_t)view * n + i0);
-        for (uint32_t q = (uint32_t)tid; q < nrec * 8u; q += 256u) {
+        const uint32_t here = nrec > 128u * half ? min(128u, nrec - 128u * half) : 0u;
+        float4* dst = reinterpret_cast<float4*>(recs + (size_t)view * n + i0 + 128u * half);
+        for (uint32_t q = tid; q < here * 8u; q += 256u) {
             const uint32_t r = q >> 3, fld = q & 7u;
-            if (s_write[r] == 0u || (fld == 4u && !write_normal)) continue;
+            if (s_write[r] == 0u) continue;
             const float4 v = s_stage[r * kRecRow + fld];
             typedef float f4v __attribute__((ext_vector_type(4)));
             __builtin_nontemporal_store(f4v{v.x, v.y, v.z, v.w}, reinterpret_cast<f4v*>(dst + q));
@@ -286,15 +228,14 @@ hipError_t launch_project(hipStream_t st, const CamParams* cams_dev, uint32_t n_
                           const float* opac, const float* sh, Record* recs, uint4* rects,
                           uint32_t* depth_keys, uint32_t* counts, uint32_t* ranges_to_clear,
                           uint32_t num_ranges, uint32_t* presort_keys, uint32_t* presort_vals,
-                          uint32_t* item_count, bool clip_to_box, uint4* emit_info, bool pack_counts,
-                          bool write_normal) {
+                          uint32_t* item_count, bool clip_to_box, uint4* emit_info, bool pack_counts) {
     if (n == 0 && num_ranges == 0 && item_count == nullptr) return hipSuccess;
     if (n_views == 0) return hipSuccess;
     const uint32_t blocks = div_up(n > num_ranges ? (n ? n : 1) : num_ranges, 256);
     dim3 grid(blocks * n_views);
     hipLaunchKernelGGL(project_kernel, grid, dim3(256), 0, st, cams_dev, n_views, n, pos, scales, quats, opac,
                        sh, recs, rects, depth_keys, counts, ranges_to_clear, num_ranges, presort_keys,
-                       presort_vals, item_count, clip_to_box, emit_info, pack_counts, write_normal);
+                       presort_vals, item_count, clip_to_box, emit_info, pack_counts);
     return hipGetLastError();
 }
 

@@ -845,13 +845,12 @@ struct RasterCore {
             const bool packed = items < (1u << (32 - kPackBits)) && shape.tile >= 16;
             GS_CHECK(P.mark(st, GS_STAGE_PROJECT));
             // Lean (trainer): with packed counts nothing downstream reads the
-            // rects, depth keys or counts, and colour-only passes never read
-            // the records' normal / depth.
+            // rects, depth keys or counts.
             const bool skip = lean && packed;
             GS_HIP(launch_project(st, cd, nv, n, pos, sc, q, op, sh, recs, skip ? nullptr : rects,
                                   skip ? nullptr : depth_keys, skip ? nullptr : offsets, ranges, 2 * max_tile_id,
                                   pre_keys[0], pre_vals[0], item_count, binning == GS_BINNING_TIGHT, emit_info,
-                                  packed, aux_outputs));
+                                  packed));
             keys_lean = skip;
             GS_CHECK(P.mark(st, GS_STAGE_SORT));
             int alt = 0;
