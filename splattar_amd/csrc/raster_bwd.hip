@@ -757,30 +757,39 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(float4* __restrict__ g
 // have. A workgroup is four waves, one per 8x8 block; nothing is summed over
 // pixels here, so each 16-lane row walks its own list of the records that
 // reach its 4x4 sub-block: a list is about a third of the tile's, and a
-// record's step has 45 instructions against ~270 with gradients and their
+// record's step has 45 instructions against ~230 with gradients and their
 // reduction, which is what shortens the critical path. 250k surfels at 1283 x
-// 717: 108 us for the state pass and 332 us for the gradient pass, where the
-// gradient pass over whole lists takes 1042 us (its longest list); 200k
-// surfels in six 640 x 360 views: 321 + 811 against 2085 us. Where no list is
-// longer than a segment (1M surfels, four 1080p views) the pass is 5 us.
+// 717: 83 us for the state pass and 190 us for the gradient pass, where a
+// gradient pass over whole lists took 1042 us (its longest list); 200k surfels
+// in six 640 x 360 views: 220 + 610 against 2085 us. Where no list is longer
+// than a segment (1M surfels, four 1080p views) the pass is 10 us.
+// Batches of 256 records that do not stop at segment boundaries, staged one
+// record a thread: 281 -> 220 us for the six views, 105 -> 71 us with aux (20k
+// surfels at 321 x 243), 92 -> 83 us for the 1283 x 717 one, against batches of
+// a segment (at most 128, two threads a record).
+// Waves per SIMD: 220 us for the six views above at five, 235 at four, 295 at
+// six (19 spilled registers); with aux 71 us at four, 84 at five.
 template <bool AUX>
-__global__ __launch_bounds__(256) void raster_state_kernel(
+constexpr uint32_t kStateWaves = AUX ? 4 : 5;
+
+template <bool AUX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStateWaves<AUX>))) void raster_state_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in, bool cull,
     uint32_t total_tiles, TileQueue queue, BwdSegments sg) {
-    constexpr int BATCH = 128;               // records staged at a time, two threads each
+    constexpr int BATCH = 256;               // records staged at a time, one a thread
     __shared__ float4 s_rec[4][BATCH];       // M Nt | A px | B py | colour opacity
     __shared__ float4 s_n[AUX ? BATCH : 1];
-    __shared__ uint8_t s_mask[BATCH][4];     // per sub-block line: the columns the record reaches
-    __shared__ uint8_t s_list[16][BATCH];
+    __shared__ uint16_t s_mask[BATCH];       // bit 4 r + c: sub-block (c, r)
+    __shared__ uint16_t s_list[16][BATCH / 2 + 1];  // slots, two a word, last record first; read one word ahead
     __shared__ uint32_t s_last[4], s_base;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Row g of wave w: sub-block (2 (w & 1) + (g & 1), 2 (w >> 1) + (g >> 1)),
     // lane p its pixel (p & 3, p >> 2).
     const int g = lane >> 4, p = lane & 15;
     const int sc = 2 * (wave & 1) + (g & 1), sr = 2 * (wave >> 1) + (g >> 1);
-    const int slot = tid >> 1, part = tid & 1;
-    uint8_t* const my_list = s_list[sr * 4 + sc];
+    const uint64_t gt_mask = (lane == 63) ? 0ull : (~0ull << (lane + 1));
+    const uint16_t* const my_list = s_list[sr * 4 + sc];
     // The pixel's index within the stored state: block, then row-major.
     const uint32_t pixel = (uint32_t)(wave * 64 + ((4 * (g >> 1) + (p >> 2)) * 8 + 4 * (g & 1) + (p & 3)));
     const uint32_t seg_len = sg.ctl[1];
@@ -797,8 +806,12 @@ __global__ __launch_bounds__(256) void raster_state_kernel(
         load_pixel<AUX>(ps, cam, (int)x0 + 4 * sc + (p & 3), (int)y0 + 4 * sr + (p >> 2), in, lambda);
         uint32_t row_last = ps.last;
         for (int o = 8; o >= 1; o >>= 1) row_last = max(row_last, (uint32_t)__shfl_xor((int)row_last, o));
-        uint32_t wave_last = row_last;
-        for (int o = 32; o >= 16; o >>= 1) wave_last = max(wave_last, (uint32_t)__shfl_xor((int)wave_last, o));
+        uint32_t rows_last[4], wave_last = 0;  // of the wave's rows
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            rows_last[q] = (uint32_t)__builtin_amdgcn_readlane((int)row_last, 16 * q);
+            wave_last = max(wave_last, rows_last[q]);
+        }
         if (lane == 0) s_last[wave] = wave_last;
         __syncthreads();
         const uint32_t maxlast =
@@ -816,55 +829,82 @@ __global__ __launch_bounds__(256) void raster_state_kernel(
             sg.table[at + k] = make_uint2(room ? gtile : ~0u, k + 1 == nseg ? k | kSegmentLast : k);
         if (tid == 0 && room) sg.split[gtile] = 1u;
         if (!room) continue;  // walked whole by the gradient pass
-        for (uint32_t s = nseg - 1; s >= 1; --s) {
-            const uint32_t k0 = s * seg_len, k1 = min(maxlast, k0 + seg_len);
-            const int nbatch = (int)((k1 - k0 + BATCH - 1) / BATCH);
-            for (int b = nbatch - 1; b >= 0; --b) {
-                const uint32_t first = k0 + (uint32_t)b * BATCH;
-                const uint32_t cnt = min((uint32_t)BATCH, k1 - first);
-                __syncthreads();  // the previous walk has read the staged records
-                if ((uint32_t)slot < cnt) {
-                    const Record* src = recs + payloads[start + first + slot];
-                    const float4* f4 = reinterpret_cast<const float4*>(src);
-                    const float4 box = src->box, e0 = src->ell0, e1 = src->ell1;
-                    const float cx = src->a_px.w, cy = src->b_py.w;
-                    s_rec[2 * part][slot] = f4[2 * part];
-                    s_rec[2 * part + 1][slot] = f4[2 * part + 1];
-                    if (AUX && part == 0) s_n[slot] = src->nrm_dep;
-                    const SubTest t = sub_test(box, e0, e1, cx, cy);
+        // The batches do not follow the segments: a row stores its pixels'
+        // state whenever its walk passes a boundary (`bound`, the first record
+        // of segment `s`).
+        uint32_t s = nseg - 1, bound = s * seg_len;
+        for (uint32_t top = maxlast; top > seg_len;) {
+            const uint32_t first = top - seg_len > (uint32_t)BATCH ? top - BATCH : seg_len, cnt = top - first;
+            __syncthreads();  // the previous walk has read the staged records
+            if ((uint32_t)tid < cnt) {
+                const Record& r = recs[payloads[start + first + (uint32_t)tid]];
+                const float4 a = r.a_px, b = r.b_py;
+                s_rec[0][tid] = r.m_nt;
+                s_rec[1][tid] = a;
+                s_rec[2][tid] = b;
+                s_rec[3][tid] = r.col_op;
+                if (AUX) s_n[tid] = r.nrm_dep;
+                uint32_t mask = 0xFFFFu;
+                if (cull) {
+                    const SubTest t = sub_test(r.box, r.ell0, r.ell1, a.w, b.w);
+                    mask = 0;
 #pragma unroll
-                    for (int r = 0; r < 2; ++r) {
-                        const int row = 2 * part + r;
-                        s_mask[slot][row] = cull ? (uint8_t)sub_row_mask(t, (float)x0, (float)(y0 + 4 * row)) : 0xFu;
+                    for (int i = 0; i < 4; ++i) mask |= sub_row_mask(t, (float)x0, (float)(y0 + 4 * i)) << 4 * i;
+                }
+                s_mask[tid] = (uint16_t)mask;
+            }
+            __syncthreads();
+            if (wave_last > first) {
+                // The wave's four lists, last record first: the records that
+                // reach a row's sub-block before its last contributor.
+                uint32_t n[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int c = BATCH / 64 - 1; c >= 0; --c) {
+                    if ((uint32_t)(c * 64) >= cnt) continue;
+                    const uint32_t slot = (uint32_t)(c * 64 + lane), mask = slot < cnt ? s_mask[slot] : 0u;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int sub = (2 * (wave >> 1) + (q >> 1)) * 4 + 2 * (wave & 1) + (q & 1);
+                        const bool hit = (mask >> sub & 1u) && first + slot < rows_last[q];
+                        const uint64_t bal = __ballot(hit);
+                        if (hit) ((uint8_t*)s_list[sub])[n[q] + (uint32_t)__popcll(bal & gt_mask)] = (uint8_t)slot;
+                        n[q] += (uint32_t)__popcll(bal);
                     }
                 }
-                __syncthreads();
-                // Each row's list, in batch order: the records that reach its
-                // sub-block before its last contributor.
-                uint32_t count = 0;
-                for (uint32_t k = 0; k < cnt; k += 16) {
-                    const uint32_t j = k + (uint32_t)p;
-                    const bool in_list =
-                        j < cnt && first + j < row_last && ((s_mask[min(j, cnt - 1)][sr] >> sc) & 1u);
-                    const uint32_t bal = (uint32_t)(__ballot(in_list) >> (16 * g)) & 0xFFFFu;
-                    if (in_list) my_list[count + (uint32_t)__popc(bal & ((1u << p) - 1u))] = (uint8_t)j;
-                    count += (uint32_t)__popc(bal);
-                }
-                __builtin_amdgcn_wave_barrier();
-                for (int kk = (int)count - 1; kk >= 0; --kk) {
-                    const uint32_t j = my_list[kk];
-                    Record r;
+                const uint32_t mine = g == 0 ? n[0] : g == 1 ? n[1] : g == 2 ? n[2] : n[3];
+                auto load = [&](uint32_t j, Record& r) {
                     r.m_nt = s_rec[0][j];
                     r.a_px = s_rec[1][j];
                     r.b_py = s_rec[2][j];
                     r.col_op = s_rec[3][j];
                     r.nrm_dep = AUX ? s_n[AUX ? j : 0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    const HitEval h = eval_hit(r, ps.sx, ps.sy, ps.pxc, ps.pyc);
-                    step_state<AUX>(ps, r, h, first + j < ps.last && h.hit, lambda);
+                };
+                auto step = [&](uint32_t rel, const Record& r, const HitEval& h) {
+                    while (rel < bound) {
+                        store_state<AUX>(sg, at + s - 1, pixel, ps);
+                        --s;
+                        bound -= seg_len;
+                    }
+                    step_state<AUX>(ps, r, h, (rel < ps.last) & h.hit, lambda);
+                };
+                // Two records a round: their evaluations do not depend on the
+                // walk state and overlap. Past a row's end: old slots, unused.
+                uint32_t jj = my_list[0];
+                for (uint32_t k = 0; __any(k < mine); k += 2) {
+                    const uint32_t j0 = jj & 0xFFu, j1 = jj >> 8;
+                    Record r0, r1;
+                    load(j0, r0);
+                    load(j1, r1);
+                    jj = my_list[k / 2 + 1];
+                    const HitEval h0 = eval_hit(r0, ps.sx, ps.sy, ps.pxc, ps.pyc);
+                    const HitEval h1 = eval_hit(r1, ps.sx, ps.sy, ps.pxc, ps.pyc);
+                    if (k < mine) step(first + j0, r0, h0);
+                    if (k + 1 < mine) step(first + j1, r1, h1);
                 }
             }
-            store_state<AUX>(sg, at + s - 1, pixel, ps);
+            top = first;
         }
+        for (; s >= 1; --s) store_state<AUX>(sg, at + s - 1, pixel, ps);
         __syncthreads();  // s_last and s_base are rewritten by the next tile
     }
 }
@@ -908,7 +948,9 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
            tile_begin, sg);
     };
     if (sg.state != nullptr) {
-        const uint32_t g = std::min(total_tiles, std::max(queue.grid_blocks / 2, 1u));
+        // As many workgroups (four waves) as the CUs hold.
+        const uint32_t fit = queue.cus * (aux ? kStateWaves<true> : kStateWaves<false>);
+        const uint32_t g = std::min(total_tiles, std::max(fit != 0u ? fit : queue.grid_blocks / 2, 1u));
         if (aux)
             hipLaunchKernelGGL(raster_state_kernel<true>, dim3(g), dim3(256), 0, st, cams_dev, n_views, ranges,
                                payloads, recs, in, cull, total_tiles, queue, sg);
