@@ -137,7 +137,7 @@ __device__ __forceinline__ uint32_t select_set_bit(uint32_t lo, uint32_t hi, uin
 // SPREAD: per_wave items a wave (a power of two) instead of 64.
 template <bool SPREAD>
 __global__ __launch_bounds__(256) void emit_tile_keys_kernel(
-    uint32_t n_items, const uint32_t* __restrict__ order, bool packed, const uint4* __restrict__ emit_info,
+    uint32_t n_items, const uint32_t* __restrict__ count, const uint32_t* __restrict__ order, bool packed, const uint4* __restrict__ emit_info,
     const uint32_t* __restrict__ offsets_sorted, const CamParams* __restrict__ cams,
     uint32_t items_per_view, uint32_t* __restrict__ tkeys, uint32_t* __restrict__ payloads,
     uint32_t max_entries, const uint32_t* __restrict__ total, uint32_t* __restrict__ sort_count,
@@ -149,6 +149,7 @@ __global__ __launch_bounds__(256) void emit_tile_keys_kernel(
         *sort_count = t < max_entries ? t : max_entries;
         if (t > max_entries) atomicOr(overflow_flag, 1u);
     }
+    n_items = min(n_items, *count);
     const int lane = threadIdx.x & 63;
     const uint32_t wave_first = (thread >> 6) * (uint32_t)per_wave, gid = wave_first + (uint32_t)lane;
     if (wave_first >= n_items) return;
@@ -338,7 +339,7 @@ hipError_t launch_tile_ranges(hipStream_t st, const uint64_t* keys, const uint32
     return hipGetLastError();
 }
 
-hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_t* order, bool packed,
+hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_t* count, const uint32_t* order, bool packed,
                                  const uint4* emit_info, const uint32_t* offsets_sorted,
                                  const CamParams* cams_dev, uint32_t items_per_view, uint32_t* tkeys,
                                  uint32_t* payloads, uint32_t max_entries, const uint32_t* total,
@@ -351,7 +352,7 @@ hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_
     while (per_wave > 4 && n_items / (uint32_t)per_wave < 2048u) per_wave /= 2;
     const uint32_t blocks = div_up(n_items > 0 ? n_items : 1, 4 * per_wave);
     auto* kernel = per_wave == 64 ? emit_tile_keys_kernel<false> : emit_tile_keys_kernel<true>;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, n_items, order, packed, emit_info, offsets_sorted,
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, n_items, count, order, packed, emit_info, offsets_sorted,
                        cams_dev, items_per_view > 0 ? items_per_view : 1, tkeys, payloads, max_entries, total,
                        sort_count, overflow_flag, per_wave);
     return hipGetLastError();

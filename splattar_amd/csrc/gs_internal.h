@@ -636,9 +636,11 @@ constexpr size_t scan_scratch_size(uint32_t capacity) {
 }
 size_t scan_scratch_bytes(uint32_t capacity);
 // Exclusive scan of in[0..n) (in place allowed), of in[perm[i]] (gather),
-// or, with in == nullptr, of perm[i] & kPackMask (packed tile counts).
+// or, with in == nullptr, of perm[i] & kPackMask (packed tile counts). With
+// count, of the first min(n, *count) items only.
 hipError_t launch_exclusive_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n,
-                                 uint32_t* total_out, void* scratch, const uint32_t* perm = nullptr);
+                                 uint32_t* total_out, void* scratch, const uint32_t* perm = nullptr,
+                                 const uint32_t* count = nullptr);
 
 // binning.hip
 hipError_t launch_emit_keys(hipStream_t st, uint32_t n_items, const uint4* rects,
@@ -653,10 +655,10 @@ hipError_t launch_fill_u32(hipStream_t st, uint32_t* dst, uint32_t value, size_t
 // dst[0..count) = src[0..count) as a kernel on the stream (device to device).
 hipError_t launch_copy_u32(hipStream_t st, uint32_t* dst, const uint32_t* src, size_t count);
 hipError_t launch_count_tiles(hipStream_t st, uint32_t n, const uint4* rects, uint32_t* counts);
-// Depth-ordered emission: order[k] is the k-th item in depth order (shifted
+// Depth-ordered emission of the first min(n_items, *count) items: order[k] is the k-th item in depth order (shifted
 // left by kPackBits over its tile count when packed), emit_info the per-item record
 // written by launch_project.
-hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_t* order, bool packed,
+hipError_t launch_emit_tile_keys(hipStream_t st, uint32_t n_items, const uint32_t* count, const uint32_t* order, bool packed,
                                  const uint4* emit_info, const uint32_t* offsets_sorted,
                                  const CamParams* cams_dev, uint32_t items_per_view, uint32_t* tkeys,
                                  uint32_t* payloads, uint32_t max_entries, const uint32_t* total,

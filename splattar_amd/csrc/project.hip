@@ -58,7 +58,8 @@ __global__ __launch_bounds__(256) void project_kernel(
         if (rects) rects[g] = rect;
         if (depth_keys) depth_keys[g] = key;
         if (counts) counts[g] = count;
-        if (presort_keys) presort_keys[g] = key;
+        // Items without entries are left out by the presort's first pass.
+        if (presort_keys) presort_keys[g] = count != 0u ? key : kDropKey;
         if (presort_vals) presort_vals[g] = pack_counts ? (g << kPackBits) | count : g;
         if (emit_info)
             emit_info[g] = make_uint4(rect.x | (rect.y << 16), rect.z | (rect.w << 16), (uint32_t)mask,

@@ -739,7 +739,7 @@ struct RasterCore {
         }
         GS_CHECK(dalloc(&offs_sorted, nv, "presorted offsets"));
         GS_CHECK(dalloc(&emit_info, nv, "emit info"));
-        GS_CHECK(dalloc(&item_count, 1, "item count"));
+        GS_CHECK(dalloc(&item_count, 2, "item counts"));
         GS_CHECK(dalloc(&ranges, (size_t)tiles * 2, "ranges"));
         GS_CHECK(dalloc(&out_color, pixels, "out_color"));
         GS_CHECK(dalloc(&out_aux, pixels, "out_aux"));
@@ -853,15 +853,18 @@ struct RasterCore {
                                   packed));
             keys_lean = skip;
             GS_CHECK(P.mark(st, GS_STAGE_SORT));
+            // Items without entries (culled, or past a view's surfels) end here:
+            // the later passes, the scan and the emission take *kept items.
+            uint32_t* const kept = item_count + 1;
             int alt = 0;
             GS_HIP(launch_radix_sort_u32(st, pre_keys[0], pre_vals[0], pre_keys[1], pre_vals[1],
-                                         item_count, items, 0, 32, digit_bits, sort_scratch, &alt));
+                                         item_count, items, 0, 32, digit_bits, sort_scratch, &alt, kept));
             const uint32_t* order = pre_vals[alt];
             GS_CHECK(P.mark(st, GS_STAGE_SCAN));
             GS_HIP(launch_exclusive_scan(st, packed ? nullptr : offsets, offs_sorted, items, total + v0,
-                                         scan_scratch, order));
+                                         scan_scratch, order, kept));
             GS_CHECK(P.mark(st, GS_STAGE_EMIT));
-            GS_HIP(launch_emit_tile_keys(st, items, order, packed, emit_info, offs_sorted, cd, n ? n : 1,
+            GS_HIP(launch_emit_tile_keys(st, items, kept, order, packed, emit_info, offs_sorted, cd, n ? n : 1,
                                          tkeys[0], pays[0], cap_entries, total + v0, sort_count + v0,
                                          overflow));
             GS_CHECK(P.mark(st, GS_STAGE_SORT));

@@ -65,11 +65,13 @@ __device__ __forceinline__ void load_run(const uint32_t* in, const uint32_t* per
 // Sum of partition blockIdx.x. With `stage`, the (gathered) values are also
 // stored there contiguously, so the second read needs no gather.
 __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* in, uint32_t n,
+                                                                   const uint32_t* __restrict__ count,
                                                                    const uint32_t* __restrict__ perm,
                                                                    uint32_t* __restrict__ stage,
                                                                    ScanScratch* __restrict__ sc) {
     __shared__ uint32_t s_wave[kScanThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (count != nullptr) n = min(n, *count);
     uint32_t v[kScanItems];
     const uint32_t first = blockIdx.x * kScanPart + (uint32_t)tid * kScanItems;
     load_run(in, perm, n, first, v);
@@ -136,10 +138,12 @@ __global__ __launch_bounds__(kSumThreads) void scan_sums_kernel(ScanScratch* __r
 // against 13; with twice the items in two rounds 12.8 against 13.8).
 constexpr uint32_t kScanSmall = kSumThreads * kScanItems;
 __global__ __launch_bounds__(kSumThreads) void scan_small_kernel(const uint32_t* in, uint32_t* out, uint32_t n,
+                                                                 const uint32_t* __restrict__ count,
                                                                  const uint32_t* __restrict__ perm,
                                                                  uint32_t* __restrict__ total) {
     __shared__ uint32_t s_wave[kSumThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (count != nullptr) n = min(n, *count);
     const uint32_t first = (uint32_t)tid * kScanItems;
     uint32_t v[kScanItems], sum = 0;
     load_run(in, perm, n, first, v);
@@ -169,11 +173,13 @@ __global__ __launch_bounds__(kSumThreads) void scan_small_kernel(const uint32_t*
 // those before its own and the last one writes the grand total, which saves
 // the launch between.
 __global__ __launch_bounds__(kScanThreads) void scan_down_kernel(const uint32_t* in, uint32_t* out, uint32_t n,
+                                                                 const uint32_t* __restrict__ count,
                                                                  const uint32_t* __restrict__ perm,
                                                                  const ScanScratch* __restrict__ sc,
                                                                  uint32_t* __restrict__ total) {
     __shared__ uint32_t s_wave[kScanThreads / 64], s_before[kScanThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (count != nullptr) n = min(n, *count);
     const uint32_t part = blockIdx.x;
     const uint32_t first = part * kScanPart + (uint32_t)tid * kScanItems;
     const uint32_t* sums = reinterpret_cast<const uint32_t*>(sc + 1);
@@ -218,7 +224,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_down_kernel(const uint32_t*
 size_t scan_scratch_bytes(uint32_t capacity) { return scan_scratch_size(capacity); }
 
 hipError_t launch_exclusive_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n,
-                                 uint32_t* total_out, void* scratch, const uint32_t* perm) {
+                                 uint32_t* total_out, void* scratch, const uint32_t* perm,
+                                 const uint32_t* count) {
     ScanScratch* sc = static_cast<ScanScratch*>(scratch);
     const uint32_t parts = (n + kScanPart - 1) / kScanPart;
     // A gather (in[perm[i]]; in and out distinct) runs once: the first pass
@@ -226,10 +233,11 @@ hipError_t launch_exclusive_scan(hipStream_t st, const uint32_t* in, uint32_t* o
     const bool gather = perm != nullptr && in != nullptr;
     hipError_t e = hipSuccess;
     if (n <= kScanSmall) {
-        hipLaunchKernelGGL(scan_small_kernel, dim3(1), dim3(kSumThreads), 0, st, in, out, n, perm, total_out);
+        hipLaunchKernelGGL(scan_small_kernel, dim3(1), dim3(kSumThreads), 0, st, in, out, n, count, perm,
+                           total_out);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(scan_reduce_kernel, dim3(parts), dim3(kScanThreads), 0, st, in, n, perm,
+    hipLaunchKernelGGL(scan_reduce_kernel, dim3(parts), dim3(kScanThreads), 0, st, in, n, count, perm,
                        gather ? out : nullptr, sc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const bool scanned = parts > (uint32_t)kScanThreads;
@@ -238,7 +246,7 @@ hipError_t launch_exclusive_scan(hipStream_t st, const uint32_t* in, uint32_t* o
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     hipLaunchKernelGGL(scan_down_kernel, dim3(parts), dim3(kScanThreads), 0, st, gather ? out : in, out, n,
-                       gather ? nullptr : perm, sc, scanned ? nullptr : total_out);
+                       count, gather ? nullptr : perm, sc, scanned ? nullptr : total_out);
     return hipGetLastError();
 }
 
