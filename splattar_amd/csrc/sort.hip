@@ -151,19 +151,22 @@ __global__ __launch_bounds__(kSortThreads) void upsweep_kernel(const K* __restri
     __shared__ uint32_t s_h[kSortWaves][R];
     const int tid = threadIdx.x;
     const uint32_t n = min(*count, cap);
-    const uint32_t part = blockIdx.x, items = sort_items(n), base = part * kSortThreads * items;
-    if (part >= sort_parts(n)) return;  // grid sized for the capacity
-    for (uint32_t k = tid; k < kSortWaves * R; k += kSortThreads) (&s_h[0][0])[k] = 0u;
-    if (items == 2) upsweep_part<K, RB, 2>(kin, n, base, shift, drop, s_h);
-    else if (items == 4) upsweep_part<K, RB, 4>(kin, n, base, shift, drop, s_h);
-    else upsweep_part<K, RB, 8>(kin, n, base, shift, drop, s_h);
-    __syncthreads();
-    uint32_t* off = part_offsets(sc);
-    for (uint32_t k = tid; k < R; k += kSortThreads) {
-        uint32_t c = 0;
+    const uint32_t items = sort_items(n), parts = sort_parts(n);
+    for (uint32_t part = blockIdx.x; part < parts; part += gridDim.x) {
+        const uint32_t base = part * kSortThreads * items;
+        for (uint32_t k = tid; k < kSortWaves * R; k += kSortThreads) (&s_h[0][0])[k] = 0u;
+        if (items == 2) upsweep_part<K, RB, 2>(kin, n, base, shift, drop, s_h);
+        else if (items == 4) upsweep_part<K, RB, 4>(kin, n, base, shift, drop, s_h);
+        else upsweep_part<K, RB, 8>(kin, n, base, shift, drop, s_h);
+        __syncthreads();
+        uint32_t* off = part_offsets(sc);
+        for (uint32_t k = tid; k < R; k += kSortThreads) {
+            uint32_t c = 0;
 #pragma unroll
-        for (int w = 0; w < kSortWaves; ++w) c += s_h[w][k];
-        off[(size_t)k * stride + part] = c;
+            for (int w = 0; w < kSortWaves; ++w) c += s_h[w][k];
+            off[(size_t)k * stride + part] = c;
+        }
+        __syncthreads();  // s_h is cleared for the next partition
     }
 }
 
@@ -537,14 +540,17 @@ hipError_t radix_sort_passes(hipStream_t st, K* (&kb)[2], uint32_t* (&vb)[2], co
         return hipGetLastError();
     }
     const bool fused = cap <= kFusedCap;
+    // A capacity far above the count launches workgroups that only leave (0.2
+    // ns each): the upsweep takes partitions past 8192 workgroups in turn; in
+    // the downsweep that loop costs 30 registers, and with them waves.
     const uint32_t grid = most_parts(cap), stride = grid;
     hipError_t e = hipSuccess;
     for (uint32_t p = 0; p < passes; ++p) {
         const uint32_t shift = begin_bit + p * RB;
         const int src = (int)(p & 1u), dst = 1 - src;
         const bool drop = kept != nullptr && p == 0;
-        hipLaunchKernelGGL((upsweep_kernel<K, RB>), dim3(grid), dim3(kSortThreads), 0, st, kb[src], count, cap, shift,
-                           stride, drop, sc);
+        hipLaunchKernelGGL((upsweep_kernel<K, RB>), dim3(std::min(grid, 8192u)), dim3(kSortThreads), 0, st, kb[src],
+                           count, cap, shift, stride, drop, sc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (!fused) {
             hipLaunchKernelGGL(part_scan_kernel, dim3(1u << RB), dim3(256), 0, st, count, cap, stride, p, 1u << RB,

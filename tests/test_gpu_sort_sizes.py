@@ -47,3 +47,19 @@ def test_sort_sizes(gpu, bits, cap, counts, digit):
         _check(s, n, bits, 4, 20, digit, 1)                # one key: the input order stays
         _check(s, n, bits, 3, 19, digit, 0xFFFFFFFF)       # whole digits: bits outside the range are ignored
     s.close()
+
+
+def test_sort_more_partitions_than_the_upsweep_has_workgroups(gpu):
+    import splattar_amd as sa
+    n = 8192 * 4096 + 5
+    announce(f"sort32 n={n}")
+    s = sa.RadixSorter(gpu, n, key_bits=32)
+    keys = oracle.xorshift32(99, n, 1 << 16)
+    s.keys().write(keys)
+    s.payloads().write(np.arange(n, dtype=np.uint32))
+    s.counts().write(np.array([n], np.uint32))
+    s.encode(end_bit=16)
+    order = np.argsort(keys.astype(np.uint16), kind="stable")
+    assert np.array_equal(s.keys().read(n), keys[order])
+    assert np.array_equal(s.payloads().read(n), order.astype(np.uint32))
+    s.close()
