@@ -679,10 +679,14 @@ hipError_t launch_compose_keys(hipStream_t st, const uint32_t* tkeys, const uint
 
 // sort.hip
 size_t sort_scratch_bytes(uint32_t capacity);
+// exact: the keys have no bits at or past end_bit, so digits may be of any
+// width; radix_sort_passes tells how many passes a sort of `bits` bits takes
+// (the result is in the alternate buffers after an odd number).
+uint32_t radix_sort_passes(uint32_t capacity, uint32_t bits, uint32_t digit_bits, bool exact);
 hipError_t launch_radix_sort_u64(hipStream_t st, uint64_t* keys0, uint32_t* vals0, uint64_t* keys1,
                                  uint32_t* vals1, const uint32_t* count, uint32_t capacity,
                                  uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
-                                 void* scratch, int* result_in_alt);
+                                 void* scratch, int* result_in_alt, bool exact = false);
 hipError_t launch_copy_pairs(hipStream_t st, const void* src_keys, const uint32_t* src_vals,
                              void* dst_keys, uint32_t* dst_vals, uint32_t key_bytes,
                              const uint32_t* count, uint32_t capacity);
@@ -692,7 +696,8 @@ constexpr uint32_t kDropKey = 0xFFFFFFFFu;
 hipError_t launch_radix_sort_u32(hipStream_t st, uint32_t* keys0, uint32_t* vals0, uint32_t* keys1,
                                  uint32_t* vals1, const uint32_t* count, uint32_t capacity,
                                  uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
-                                 void* scratch, int* result_in_alt, uint32_t* kept = nullptr);
+                                 void* scratch, int* result_in_alt, bool exact = false,
+                                 uint32_t* kept = nullptr);
 // The order of launch_tile_order_keys, sorted, in one launch: up to
 // tile_order_small_cap() tiles.
 uint32_t tile_order_small_cap();

@@ -502,16 +502,15 @@ gs_status gs_binner_encode(gs_binner b, void* stream, uint32_t num_items, uint32
     }
     GS_HIP(launch_count_tiles(st, num_items, b->rects, b->offsets));
     GS_HIP(launch_exclusive_scan(st, b->offsets, b->offsets, num_items, b->total, b->scan_scratch));
-    GS_HIP(launch_emit_keys(st, num_items, b->rects, b->depths, b->offsets, b->cam,
-                            num_items ? num_items : 1, tiles_x, b->keys[0], b->vals[0],
-                            b->max_entries, b->total, b->count, b->overflow));
+    // Emitted into the buffers from which the sort's passes end in the first.
     const uint32_t end_bit = 32 + bits_for(b->num_tiles);
+    const uint32_t src = radix_sort_passes(b->max_entries, end_bit, digit_bits, true) & 1u;
+    GS_HIP(launch_emit_keys(st, num_items, b->rects, b->depths, b->offsets, b->cam,
+                            num_items ? num_items : 1, tiles_x, b->keys[src], b->vals[src],
+                            b->max_entries, b->total, b->count, b->overflow));
     int alt = 0;
-    GS_HIP(launch_radix_sort_u64(st, b->keys[0], b->vals[0], b->keys[1], b->vals[1], b->count,
-                                 b->max_entries, 0, end_bit, digit_bits, b->sort_scratch, &alt));
-    if (alt)
-        GS_HIP(launch_copy_pairs(st, b->keys[1], b->vals[1], b->keys[0], b->vals[0], 8, b->count,
-                                 b->max_entries));
+    GS_HIP(launch_radix_sort_u64(st, b->keys[src], b->vals[src], b->keys[1 - src], b->vals[1 - src], b->count,
+                                 b->max_entries, 0, end_bit, digit_bits, b->sort_scratch, &alt, true));
     GS_HIP(launch_fill_u32(st, b->ranges, 0u, (size_t)b->num_tiles * 2));  // binning.rs:228
     GS_HIP(launch_tile_ranges(st, b->keys[0], b->count, b->max_entries, b->ranges));
     return GS_OK;
@@ -858,7 +857,7 @@ struct RasterCore {
             uint32_t* const kept = item_count + 1;
             int alt = 0;
             GS_HIP(launch_radix_sort_u32(st, pre_keys[0], pre_vals[0], pre_keys[1], pre_vals[1],
-                                         item_count, items, 0, 32, digit_bits, sort_scratch, &alt, kept));
+                                         item_count, items, 0, 32, digit_bits, sort_scratch, &alt, true, kept));
             const uint32_t* order = pre_vals[alt];
             GS_CHECK(P.mark(st, GS_STAGE_SCAN));
             GS_HIP(launch_exclusive_scan(st, packed ? nullptr : offsets, offs_sorted, items, total + v0,
@@ -870,7 +869,7 @@ struct RasterCore {
             GS_CHECK(P.mark(st, GS_STAGE_SORT));
             GS_HIP(launch_radix_sort_u32(st, tkeys[0], pays[0], tkeys[1], pays[1], sort_count + v0,
                                          cap_entries, 0, bits_for(max_tile_id), digit_bits, sort_scratch,
-                                         &result_alt));
+                                         &result_alt, true));
             GS_CHECK(P.mark(st, GS_STAGE_RANGES));
             GS_HIP(launch_tile_ranges_u32(st, tkeys[result_alt], sort_count + v0, cap_entries, ranges));
             keys64_valid = false;
@@ -894,7 +893,7 @@ struct RasterCore {
         const uint32_t end_bit = 32 + bits_for(max_tile_id);
         GS_CHECK(P.mark(st, GS_STAGE_SORT));
         GS_HIP(launch_radix_sort_u64(st, keys[0], pays[0], keys[1], pays[1], sort_count + v0,
-                                     cap_entries, 0, end_bit, digit_bits, sort_scratch, &result_alt));
+                                     cap_entries, 0, end_bit, digit_bits, sort_scratch, &result_alt, true));
         GS_CHECK(P.mark(st, GS_STAGE_RANGES));
         GS_HIP(launch_tile_ranges(st, keys[result_alt], sort_count + v0, cap_entries, ranges));
         keys64_valid = true;
