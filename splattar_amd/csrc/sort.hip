@@ -21,9 +21,10 @@
 // keys and payloads in turn, 12 B a pair read, 8 written).
 // No partition waits for another (a decoupled look-back walked ~6 rounds of
 // 16 predecessor statuses per partition here and read ~1.8x the keys' bytes).
-// Digit width is 4 or 8 bits; only the bit range [begin_bit, end_bit) is
-// sorted, so a key whose high bits are known constant costs fewer passes. A
-// count above the capacity sorts the first `capacity` pairs.
+// Digit width is 4 or 8 bits (9 where the caller allows it); only the bit range
+// [begin_bit, end_bit) is sorted, so a key whose high bits are known constant
+// costs fewer passes. A count above the capacity sorts the first `capacity`
+// pairs.
 //
 // Per pass HBM traffic: read (2 sizeof(K) + 4) B and write (sizeof(K) + 4) B
 // per pair, plus 8 B per partition and digit of offsets.
