@@ -380,7 +380,8 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     static_assert(BATCH % 64 == 0 && BATCH <= (1 << MB), "batch of whole waves");
     __shared__ float4 s_m[BATCH], s_a[BATCH], s_b[BATCH], s_c[BATCH], s_n[AUX ? BATCH : 1];
     __shared__ uint32_t s_pay[BATCH];        // the batch's surfel ids, for the flush
-    __shared__ uint16_t s_list[NW][BATCH];
+    __shared__ uint16_t s_list[NW][BATCH + 1];  // read one entry ahead
+    __shared__ uint32_t s_wlast[NW][2];        // last contributors of each wave's blocks
     __shared__ uint32_t s_qcnt[SW][NW];      // [staging wave][list wave]
     // One or two waves: a copy of the slots per wave, written (a wave meets a
     // record once per batch) and summed at the flush; LDS float atomics run at
@@ -431,7 +432,11 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
         if constexpr (TWO) load_pixel<AUX>(pb, cam, px, py + 8, in, lambda);
         else pb.last = 0u;
         const uint32_t last_a = wave_max(pa.last), last_b = wave_max(pb.last);
-        if (lane == 0) atomicMax(&s_maxlast, max(last_a, last_b));
+        if (lane == 0) {
+            s_wlast[wave][0] = last_a;
+            s_wlast[wave][1] = last_b;
+            atomicMax(&s_maxlast, max(last_a, last_b));
+        }
         __syncthreads();
         const uint32_t maxlast = s_maxlast;
         if (maxlast == 0) continue;
@@ -477,8 +482,10 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
 #pragma unroll
                 for (int w = 0; w < NW; ++w) {
                     const int bt = TWO ? (2 * (w / NC)) * NC + w % NC : 0;
-                    const uint32_t top = (qmask >> bt) & 1u;
-                    const uint32_t bot = TWO ? (qmask >> (bt + NC)) & 1u : 0u;
+                    // A block is walked only from its last contributor on.
+                    const uint32_t rel = first + (uint32_t)slot;
+                    const uint32_t top = rel < s_wlast[w][0] ? (qmask >> bt) & 1u : 0u;
+                    const uint32_t bot = TWO && rel < s_wlast[w][1] ? (qmask >> (bt + NC)) & 1u : 0u;
                     memb[m][w] = top | (bot << 1);
                     const uint64_t bal = __ballot(memb[m][w] != 0u);
                     qpos[m][w] = (uint32_t)__popcll(bal & lt_mask);
@@ -500,7 +507,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                     if (memb[m][w] != 0u) {
                         uint32_t off = 0;
                         for (int v = 0; v < sw; ++v) off += s_qcnt[v][w];
-                        s_list[w][off + qpos[m][w]] = (uint16_t)(slot | (memb[m][w] << MB));
+                        s_list[w][1 + off + qpos[m][w]] = (uint16_t)(slot | (memb[m][w] << MB));
                     }
                 }
             }
@@ -509,18 +516,15 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
             for (int v = 0; v < SW; ++v) my_count += (int)s_qcnt[v][wave];
             __syncthreads();
 
-            for (int kk = my_count - 1; kk >= 0; --kk) {
+            uint32_t next = s_list[wave][my_count];
+            for (int kk = my_count; kk > 0; --kk) {
                 // The entry is the same for every lane: make it scalar, so the
                 // block branches below are uniform.
-                const uint32_t e = __builtin_amdgcn_readfirstlane((uint32_t)s_list[wave][kk]);
+                const uint32_t e = __builtin_amdgcn_readfirstlane(next);
+                next = s_list[wave][kk - 1];
                 const uint32_t j = e & ((1u << MB) - 1u);
-                const bool top = (e >> MB) & 1u, bot = TWO && ((e >> (MB + 1)) & 1u);
+                const bool need_a = (e >> MB) & 1u, need_b = TWO && ((e >> (MB + 1)) & 1u);
                 const uint32_t rel = first + j;
-                // A block is walked only while some pixel of it is at or before
-                // its last contributor (a pixel past it changes nothing).
-                const bool need_a = top && rel < last_a;
-                const bool need_b = bot && rel < last_b;
-                if (!need_a && !need_b) continue;
                 Record r;
                 r.m_nt = s_m[j];
                 r.a_px = s_a[j];
@@ -545,6 +549,8 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 if (!go_a && !go_b) continue;
                 float g[16];
                 float g2[4];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) asm volatile("" : "=v"(g[k]));  // defined here: else copied before the sums
                 g[kGNt] = 0.0f;  // written only by the AUX terms
 #pragma unroll
                 for (int k = 0; k < 4; ++k) g2[k] = 0.0f;
