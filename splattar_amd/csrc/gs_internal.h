@@ -783,7 +783,6 @@ struct BwdIn {
 // the gradient pass then takes every segment as a unit of its own. A tile's
 // walk is sequential in depth, so without this the longest list is the
 // launch's critical path. state == nullptr: off.
-constexpr uint32_t kSegmentPool = 12288;   // segments of one pass
 constexpr uint32_t kSegmentTarget = 6144;  // a segment holds at least 1 / this of the entries
 constexpr uint32_t kSegmentMin = 32;       // and at least this many records,
 constexpr uint32_t kSegmentMinAux = 64;    // with aux, whose states are three times as large
@@ -796,16 +795,19 @@ struct BwdSegments {
     float4* state = nullptr;     // [1, with aux 3][pool][kSegmentPixels]
     uint32_t pool = 0;
 };
-// Split tiles' lists are longer than a segment of at least E / kSegmentTarget
-// (E = entries) and at least kSegmentMin records, so a tile has at most 2 len
-// / L of them and all have at most 2 E / L. Measured at 6144 and 32 against
+// A segment holds L records, L a multiple of 32 of at least E / kSegmentTarget
+// rounded down (E = entries), so all lists together have at most E / L <= 33/32
+// kSegmentTarget whole segments and each split tile, longer than L, one more;
+// there are no more split tiles than E / L either.
+// Measured at 6144 and 32 against
 // half and twice the target: plain 250k 2x1283x717 1738 against 1827 / 1732 us,
 // batch 200k 6x640x360 1857 against 1965 / 1815 us, 100k eight uneven views 1557
 // against 1558 / 1642 us; a minimum of 64 loses 3 % at 10k 256px (396 against
 // 384 us) and gains 9 % with aux (20k 321x243: 483 against 531 us).
-constexpr uint32_t segment_pool(uint32_t max_entries) {
-    const uint64_t most = 2ull * max_entries / kSegmentMin + 16;
-    return (uint32_t)(most < kSegmentPool + 16 ? most : kSegmentPool + 16);
+constexpr uint32_t segment_pool(uint32_t max_entries, uint32_t tiles) {
+    constexpr uint64_t whole = kSegmentTarget + kSegmentTarget / 32 + 1;
+    const uint64_t by_entries = 2ull * max_entries / kSegmentMin, by_tiles = whole + (tiles < whole ? tiles : whole);
+    return (uint32_t)(by_entries < by_tiles ? by_entries : by_tiles) + 16;
 }
 // Clears the gradient accumulator (floats a multiple of 4) and readies a
 // backward pass: the queue's cursors (optional), the split flags of

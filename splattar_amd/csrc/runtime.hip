@@ -745,7 +745,7 @@ struct RasterCore {
         GS_CHECK(dalloc(&out_normal, pixels, "out_normal"));
         GS_CHECK(dalloc(&ncontrib, pixels, "ncontrib"));
         GS_CHECK(dalloc(&grad_coef, nv * kGradStride, "grad_coef"));
-        segs.pool = segment_pool(entries);
+        segs.pool = segment_pool(entries, tiles);
         GS_CHECK(dalloc(&segs.ctl, 2, "segment control"));
         GS_CHECK(dalloc(&segs.table, segs.pool, "segment table"));
         GS_CHECK(dalloc(&segs.split, tiles, "split tiles"));
