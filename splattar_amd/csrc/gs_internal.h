@@ -800,7 +800,7 @@ struct BwdSegments {
 // kSegmentTarget whole segments and each split tile, longer than L, one more;
 // there are no more split tiles than E / L either.
 // Measured at 6144 and 32 against
-// half and twice the target: plain 250k 2x1283x717 1738 against 1827 / 1732 us,
+// half and twice the target (250k 2x1283x717 1738 against 1827 / 1732 us),
 // batch 200k 6x640x360 1857 against 1965 / 1815 us, 100k eight uneven views 1557
 // against 1558 / 1642 us; a minimum of 64 loses 3 % at 10k 256px (396 against
 // 384 us) and gains 9 % with aux (20k 321x243: 483 against 531 us).
