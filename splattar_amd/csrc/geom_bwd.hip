@@ -102,24 +102,33 @@ __device__ __forceinline__ void zero_acc(SurfelAcc& a) {
 // Loads one view's coefficient gradients of surfel i (GS slots stored per
 // (view, surfel); the rest are 0); false when all are 0 (the surfel did not
 // reach a pixel of the view).
-template <int GS>
-__device__ __forceinline__ bool load_coef_grads(const float* __restrict__ grad_coef, uint32_t v, uint32_t n,
+template <int GS, typename Slot>
+__device__ __forceinline__ bool load_coef_grads(const Slot* __restrict__ grad_coef, uint32_t v, uint32_t n,
                                                 uint32_t i, float gc[kGradStride]) {
-    const float4* src = reinterpret_cast<const float4*>(grad_coef + ((size_t)v * n + i) * GS);
+    typedef Slot vec4 __attribute__((ext_vector_type(4)));
+    const vec4* src = reinterpret_cast<const vec4*>(grad_coef + ((size_t)v * n + i) * GS);
 #pragma unroll
     for (int k = GS; k < kGradStride; ++k) gc[k] = 0.0f;
 #pragma unroll
     for (int k = 0; k < GS / 4; ++k) {
-        const float4 t = src[k];
-        gc[4 * k + 0] = t.x;
-        gc[4 * k + 1] = t.y;
-        gc[4 * k + 2] = t.z;
-        gc[4 * k + 3] = t.w;
+        const vec4 t = src[k];
+        gc[4 * k + 0] = (float)t.x;
+        gc[4 * k + 1] = (float)t.y;
+        gc[4 * k + 2] = (float)t.z;
+        gc[4 * k + 3] = (float)t.w;
     }
     bool any = false;
 #pragma unroll
     for (int k = 0; k < GS; ++k) any |= gc[k] != 0.0f;
     return any;
+}
+
+// Adds a view's term to a sum over views, never as a fused multiply-add with
+// the term's last product: a pass over one view that adds to stored gradients
+// then rounds like a pass over all views.
+__device__ __forceinline__ void add_term(float& sum, float term) {
+#pragma clang fp contract(off)
+    sum = sum + term;
 }
 
 // Adds one view's contribution of one surfel (activated position p, scales s,
@@ -181,14 +190,12 @@ __device__ __forceinline__ void add_view(const CamParams& cam, const float gc[kG
     const V3f ax_u = v3(1.f - 2.f * (y * y + z * z), 2.f * (x * y + ww * z), 2.f * (x * z - ww * y));
     const V3f ax_v = v3(2.f * (x * y - ww * z), 1.f - 2.f * (x * x + z * z), 2.f * (y * z + ww * x));
     const V3f dy_u = rmul(dtu), dy_v = rmul(dtv);
-    a.sc[0] += dt(dy_u, ax_u);
-    a.sc[1] += dt(dy_v, ax_v);
+    add_term(a.sc[0], dt(dy_u, ax_u));
+    add_term(a.sc[1], dt(dy_v, ax_v));
     float dq[4];
     quat_grad_cols01(x, y, z, ww, f.qn, dy_u * s.x, dy_v * s.y, dq);
-    a.q[0] += dq[0];
-    a.q[1] += dq[1];
-    a.q[2] += dq[2];
-    a.q[3] += dq[3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) add_term(a.q[k], dq[k]);
     // Colour -> SH (+ view direction). The clamp mask is already applied: the
     // rasterizer backward drops the colour gradient of a channel clamped at 0.
     const V3f dcol = v3(gc[kGCol], gc[kGCol + 1], gc[kGCol + 2]);
@@ -203,10 +210,11 @@ __device__ __forceinline__ void add_view(const CamParams& cam, const float gc[kG
         for (int k = 0; k < 16; ++k) {
             sdot[k] = 0.f;
             if (k < nb) {
-                a.sh[3 * k + 0] += dcol.x * basis[k];
-                a.sh[3 * k + 1] += dcol.y * basis[k];
-                a.sh[3 * k + 2] += dcol.z * basis[k];
-                if (!VEC) sdot[k] = shp[3 * k] * dcol.x + shp[3 * k + 1] * dcol.y + shp[3 * k + 2] * dcol.z;
+                add_term(a.sh[3 * k + 0], dcol.x * basis[k]);
+                add_term(a.sh[3 * k + 1], dcol.y * basis[k]);
+                add_term(a.sh[3 * k + 2], dcol.z * basis[k]);
+                // Explicit, as below: both forms round alike.
+                if (!VEC) sdot[k] = fmaf(shp[3 * k + 2], dcol.z, fmaf(shp[3 * k], dcol.x, shp[3 * k + 1] * dcol.y));
             }
         }
         if (VEC) {
@@ -223,7 +231,9 @@ __device__ __forceinline__ void add_view(const CamParams& cam, const float gc[kG
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int m = 4 * c + j;
-                    if (m < 3 * nb) sdot[m / 3] += f[j] * dc[m % 3];
+                    if (m >= 3 * nb) continue;
+                    float& t = sdot[m / 3];
+                    t = m % 3 == 0 ? f[j] : m % 3 == 1 ? fmaf(t, dc[0], f[j] * dc[1]) : fmaf(f[j], dc[2], t);
                 }
             }
         }
@@ -233,10 +243,10 @@ __device__ __forceinline__ void add_view(const CamParams& cam, const float gc[kG
         dpos = dpos + dv;
         dcenter = dcenter - dv;
     }
-    a.pos[0] += dpos.x;
-    a.pos[1] += dpos.y;
-    a.pos[2] += dpos.z;
-    a.op += gc[kGOp];
+    add_term(a.pos[0], dpos.x);
+    add_term(a.pos[1], dpos.y);
+    add_term(a.pos[2], dpos.z);
+    add_term(a.op, gc[kGOp]);
     if (want_cam) {
         // dL/dR_cam[j][k] += y_j da_k for a = R^T y (backward.rs:252-257).
         const V3f xw = v3(f.xx, f.xy, f.xz);
@@ -258,11 +268,11 @@ __device__ __forceinline__ void add_view(const CamParams& cam, const float gc[kG
     }
 }
 
-template <int GS>
+template <int GS, typename Slot>
 __global__ __launch_bounds__(kGeomThreads) void geom_bwd_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, uint32_t n, const float4* __restrict__ pos,
     const float2* __restrict__ scales, const float4* __restrict__ quats, const float* __restrict__ sh,
-    const float* __restrict__ grad_coef, ParamGrads g,
+    const Slot* __restrict__ grad_coef, ParamGrads g,
     int accumulate, float* __restrict__ cam_partials) {
     __shared__ float s_cam[kGeomThreads / 64][16];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -366,8 +376,9 @@ __device__ __forceinline__ void adam4(const AdamClass& c, float lr, float reg, f
 
 // Table classes: 0 position (float4 rows), 1 scales (float2), 2 quaternion
 // (float4), 3 opacity, 4 SH (48 floats); checked by the launcher.
+template <typename Slot>
 __global__ __launch_bounds__(kFuseThreads, 3) void geom_adam_kernel(
-    const CamParams* __restrict__ cams, uint32_t n_views, uint32_t n, const float* __restrict__ grad_coef,
+    const CamParams* __restrict__ cams, uint32_t n_views, uint32_t n, const Slot* __restrict__ grad_coef,
     const AdamTable table, const AdamState* __restrict__ state, ParamGrads keep) {
     __shared__ float4 s_sh[kFuseThreads * kShRow];
     const uint32_t i = blockIdx.x * kFuseThreads + threadIdx.x;
@@ -487,7 +498,7 @@ __global__ __launch_bounds__(256) void cam_reduce_kernel(const float* __restrict
 }  // namespace
 
 hipError_t launch_geom_adam(hipStream_t st, const CamParams* cams_dev, uint32_t n_views, uint32_t n,
-                            const float* grad_coef, const AdamTable& table,
+                            CoefSlots grad_coef, const AdamTable& table,
                             const AdamState* state, ParamGrads keep) {
     if (n == 0) return hipSuccess;
     // The kernel's fixed class layout and row shapes.
@@ -502,8 +513,13 @@ hipError_t launch_geom_adam(hipStream_t st, const CamParams* cams_dev, uint32_t 
     }
     if (keep.pos != nullptr && (((uintptr_t)keep.sh & 15u) || !keep.scales || !keep.quat || !keep.opacity))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(geom_adam_kernel, dim3(div_up(n, kFuseThreads)), dim3(kFuseThreads), 0, st, cams_dev,
-                       n_views, n, grad_coef, table, state, keep);
+    const dim3 grid(div_up(n, kFuseThreads));
+    if (grad_coef.wide)
+        hipLaunchKernelGGL(geom_adam_kernel<double>, grid, dim3(kFuseThreads), 0, st, cams_dev, n_views, n,
+                           static_cast<const double*>(grad_coef.data), table, state, keep);
+    else
+        hipLaunchKernelGGL(geom_adam_kernel<float>, grid, dim3(kFuseThreads), 0, st, cams_dev, n_views, n,
+                           static_cast<const float*>(grad_coef.data), table, state, keep);
     return hipGetLastError();
 }
 
@@ -513,7 +529,7 @@ size_t geom_cam_partials_bytes(uint32_t n, uint32_t n_views) {
 
 hipError_t launch_geom_bwd(hipStream_t st, const CamParams* cams_dev, uint32_t n_views, uint32_t n,
                            const float4* pos, const float2* scales, const float4* quats,
-                           const float* sh, const float* grad_coef, bool aux,
+                           const float* sh, CoefSlots grad_coef, bool aux,
                            ParamGrads g, bool accumulate, float* cam_partials) {
     if (n_views == 0) return hipSuccess;
     if (n == 0) {
@@ -525,12 +541,14 @@ hipError_t launch_geom_bwd(hipStream_t st, const CamParams* cams_dev, uint32_t n
     }
     const uint32_t blocks = div_up(n, kGeomThreads);
     float* parts = g.cam ? cam_partials : nullptr;
-    if (aux)
-        hipLaunchKernelGGL(geom_bwd_kernel<grad_stride(true)>, dim3(blocks), dim3(kGeomThreads), 0, st, cams_dev,
-                           n_views, n, pos, scales, quats, sh, grad_coef, g, accumulate ? 1 : 0, parts);
-    else
-        hipLaunchKernelGGL(geom_bwd_kernel<grad_stride(false)>, dim3(blocks), dim3(kGeomThreads), 0, st, cams_dev,
-                           n_views, n, pos, scales, quats, sh, grad_coef, g, accumulate ? 1 : 0, parts);
+    if (aux && grad_coef.wide) return hipErrorInvalidValue;
+    auto launch = [&](auto* kernel, auto* slots) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kGeomThreads), 0, st, cams_dev, n_views, n, pos, scales, quats,
+                           sh, slots, g, accumulate ? 1 : 0, parts);
+    };
+    if (aux) launch(geom_bwd_kernel<grad_stride(true), float>, static_cast<const float*>(grad_coef.data));
+    else if (grad_coef.wide) launch(geom_bwd_kernel<grad_stride(false), double>, static_cast<const double*>(grad_coef.data));
+    else launch(geom_bwd_kernel<grad_stride(false), float>, static_cast<const float*>(grad_coef.data));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !parts) return e;
     hipLaunchKernelGGL(cam_reduce_kernel, dim3(n_views), dim3(256), 0, st, parts, blocks, g.cam,

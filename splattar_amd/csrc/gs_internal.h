@@ -75,6 +75,21 @@ enum GradSlot : int {
 // Slots per (view, surfel) in memory: colour-only backward passes (no depth,
 // distortion or normal terms) keep the first 16.
 constexpr int grad_stride(bool aux) { return aux ? (int)kGradStride : 16; }
+// The slots in memory. A slot is the sum of what the tiles add with atomics, in
+// whatever order they come. In f32 the order shows in the last bits, and ten
+// Adam steps later a pixel's alpha or depth decision may fall the other way, so
+// that plain, batched and graph steps of one scene part. In f64 (wide) the sum
+// rounded to f32 does not depend on the order. Wide costs twice the bytes of the
+// atomics, the clear and the geometry pass's read, so a trainer takes it up to
+// kWideSlotBytes (32768 view-surfels), where that is nothing: a step of 10k
+// surfels at 256 x 256 217 us either way, 100k at 1080p 493 us in f32 and 497 in
+// f64, 1M in four 1080p views 3335 and 3437, 1.25M in sixteen 720p 8828 and 9450.
+struct CoefSlots {
+    void* data = nullptr;  // float or, with wide, double
+    bool wide = false;
+    size_t bytes(size_t slots) const { return slots * (wide ? sizeof(double) : sizeof(float)); }
+};
+constexpr size_t kWideSlotBytes = 4u << 20;
 
 // Camera as the kernels see it (crates/gs-kernels/src/shaders/
 // raster_common.wgsl:5-20 RasterCamera), one per view.
@@ -809,15 +824,15 @@ constexpr uint32_t segment_pool(uint32_t max_entries, uint32_t tiles) {
     const uint64_t by_entries = 2ull * max_entries / kSegmentMin, by_tiles = whole + (tiles < whole ? tiles : whole);
     return (uint32_t)(by_entries < by_tiles ? by_entries : by_tiles) + 16;
 }
-// Clears the gradient accumulator (floats a multiple of 4) and readies a
+// Clears the gradient accumulator (slots a multiple of 4) and readies a
 // backward pass: the queue's cursors (optional), the split flags of
 // split_tiles tiles and the segment length for *entries entries.
-hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
+hipError_t launch_bwd_prepare(hipStream_t st, CoefSlots grad_coef, size_t slots, uint32_t* cursor, BwdSegments sg,
                               uint32_t split_tiles, const uint32_t* entries, bool aux);
 hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const CamParams* cams_host,
                              uint32_t n_views, uint32_t total_tiles, const uint32_t* ranges,
                              const uint32_t* payloads, const Record* recs, BwdIn in,
-                             float* grad_coef, bool aux, bool cull = true,
+                             CoefSlots grad_coef, bool aux, bool cull = true,
                              TileQueue queue = {nullptr, nullptr, 0}, RasterShape shape = {},
                              uint32_t tile_begin = 0, BwdSegments sg = {});
 
@@ -833,7 +848,7 @@ struct ParamGrads {
 size_t geom_cam_partials_bytes(uint32_t n, uint32_t n_views);
 hipError_t launch_geom_bwd(hipStream_t st, const CamParams* cams_dev, uint32_t n_views, uint32_t n,
                            const float4* pos, const float2* scales, const float4* quats,
-                           const float* sh, const float* grad_coef, bool aux, ParamGrads g, bool accumulate,
+                           const float* sh, CoefSlots grad_coef, bool aux, ParamGrads g, bool accumulate,
                            float* cam_partials);
 
 // loss.hip
@@ -1029,7 +1044,7 @@ hipError_t launch_adam(hipStream_t st, const AdamTable& table, uint32_t total_bl
 // surfel) (colour-only backward). hipErrorInvalidValue for any other class
 // table.
 hipError_t launch_geom_adam(hipStream_t st, const CamParams* cams_dev, uint32_t n_views, uint32_t n,
-                            const float* grad_coef, const AdamTable& table, const AdamState* state,
+                            CoefSlots grad_coef, const AdamTable& table, const AdamState* state,
                             ParamGrads keep);
 
 }  // namespace gs

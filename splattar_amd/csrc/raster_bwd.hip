@@ -14,7 +14,7 @@
 //     8x8 block (raster_bwd_wave_kernel): a record is evaluated only in the
 //     blocks its footprint reaches, its terms over the tile are summed in
 //     registers, reduced once per (record, tile) and added to the record's
-//     gradient with hardware global FP32 atomics (no CAS loops). A 32x32
+//     gradient with hardware global atomics, FP32 or FP64 (no CAS loops). A 32x32
 //     tile is eight waves, each owning an 8-wide, 16-tall column of two
 //     blocks (two pixels per lane), whose per-record reductions meet in LDS
 //     slots (ds_add_f32) flushed once per batch (the two waves of the depth /
@@ -363,11 +363,11 @@ __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitE
     }
 }
 
-template <bool AUX, int TW, int BATCH>
+template <bool AUX, int TW, int BATCH, typename Slot>
 __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in,
-    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
+    Slot* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
     BwdSegments sg) {
     constexpr int NS = grad_stride(AUX);     // slots per record (LDS and grad_coef)
     constexpr bool TWO = TW >= 16;           // two pixels per lane (an 8x16 column per wave)
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                         const float cc = slot == kGCol ? c.x : (slot == kGCol + 1 ? c.y : c.z);
                         if (cc == 0.0f) continue;
                     }
-                    atomicAdd(&grad_coef[(size_t)s_pay[e] * NS + slot], v);
+                    atomicAdd(&grad_coef[(size_t)s_pay[e] * NS + slot], (Slot)v);
                 }
             }
             __syncthreads();
@@ -603,11 +603,11 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
 // values go straight to the global FP32 atomics (no LDS accumulation slots:
 // one wave is the only contributor of its tile). The records a batch stages
 // form one order-preserving list carrying each record's 4-bit block mask.
-template <int BATCH>
+template <int BATCH, typename Slot>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void raster_bwd_wave_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in,
-    float* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
+    Slot* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
     BwdSegments sg) {
     constexpr int NS = grad_stride(false);
     constexpr int SPT = BATCH / 64;          // staging rounds per batch
@@ -730,8 +730,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ra
                 if (blocks == 0u) continue;
                 const float red = wave_sums16(g);
                 const uint64_t writers = kWriters & ~((uint64_t)(e >> 12) << (4 * kGCol));
-                float* const dst = grad_coef + (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(s_pay[j]) * NS;
-                if (__builtin_amdgcn_inverse_ballot_w64(writers) && red != 0.0f) atomicAdd(dst + (lane >> 2), red);
+                Slot* const dst = grad_coef + (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(s_pay[j]) * NS;
+                if (__builtin_amdgcn_inverse_ballot_w64(writers) && red != 0.0f) atomicAdd(dst + (lane >> 2), (Slot)red);
             }
         }
     }
@@ -915,25 +915,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStateWaves
     }
 }
 
-template <bool AUX, int TW, int BATCH>
-void launch_bwd(hipStream_t st, uint32_t grid, const CamParams* cams_dev, uint32_t n_views,
-                uint32_t total_tiles, const uint32_t* ranges, const uint32_t* payloads, const Record* recs,
-                BwdIn in, float* grad_coef, bool cull, TileQueue queue, uint32_t tile_begin, BwdSegments sg) {
-    constexpr int NT = TW == 8 ? 64 : TW * TW / 2;
-    hipLaunchKernelGGL((raster_bwd_kernel<AUX, TW, BATCH>), dim3(grid), dim3(NT), 0, st, cams_dev, n_views,
-                       ranges, payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
-}
-
 }  // namespace
 
-hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, uint32_t* cursor, BwdSegments sg,
+hipError_t launch_bwd_prepare(hipStream_t st, CoefSlots grad_coef, size_t slots, uint32_t* cursor, BwdSegments sg,
                               uint32_t split_tiles, const uint32_t* entries, bool aux) {
-    const size_t vecs = floats / 4;
-    if (floats % 4 != 0) return hipErrorInvalidValue;
+    const size_t vecs = grad_coef.bytes(slots) / sizeof(float4);
+    if (slots % 4 != 0) return hipErrorInvalidValue;
     uint64_t blocks = (std::max<size_t>(vecs, split_tiles) + 255) / 256;
     blocks = std::min<uint64_t>(std::max<uint64_t>(blocks, 1), 4096);
     hipLaunchKernelGGL(bwd_prepare_kernel, dim3((uint32_t)blocks), dim3(256), 0, st,
-                       reinterpret_cast<float4*>(grad_coef), vecs, cursor, sg, split_tiles, entries,
+                       static_cast<float4*>(grad_coef.data), vecs, cursor, sg, split_tiles, entries,
                        aux ? kSegmentMinAux : kSegmentMin);
     return hipGetLastError();
 }
@@ -941,7 +932,7 @@ hipError_t launch_bwd_prepare(hipStream_t st, float* grad_coef, size_t floats, u
 hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const CamParams* /*cams_host*/,
                              uint32_t n_views, uint32_t total_tiles, const uint32_t* ranges,
                              const uint32_t* payloads, const Record* recs, BwdIn in,
-                             float* grad_coef, bool aux, bool cull, TileQueue queue, RasterShape shape,
+                             CoefSlots grad_coef, bool aux, bool cull, TileQueue queue, RasterShape shape,
                              uint32_t tile_begin, BwdSegments sg) {
     if (total_tiles == 0) return hipSuccess;
     const uint32_t t = shape.tile, b = shape.bwd_batch;
@@ -949,9 +940,13 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
     if (queue.cursor == nullptr || t != 16) sg = BwdSegments{};
     const uint32_t most = total_tiles + (sg.state != nullptr ? sg.pool : 0u);
     const uint32_t grid = queue.cursor != nullptr ? std::min(most, std::max(queue.grid_blocks, 1u)) : total_tiles;
-    auto go = [&](auto fn) {
-        fn(st, grid, cams_dev, n_views, total_tiles, ranges, payloads, recs, in, grad_coef, cull, queue,
-           tile_begin, sg);
+    auto launch = [&](auto* kernel, auto* slots, uint32_t blocks, uint32_t threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, st, cams_dev, n_views, ranges, payloads, recs, in,
+                           slots, cull, total_tiles, queue, tile_begin, sg);
+    };
+    auto go = [&](auto* narrow, auto* wide, uint32_t blocks, uint32_t threads) {
+        if (grad_coef.wide) launch(wide, static_cast<double*>(grad_coef.data), blocks, threads);
+        else launch(narrow, static_cast<float*>(grad_coef.data), blocks, threads);
     };
     if (sg.state != nullptr) {
         // As many workgroups (four waves) as the CUs hold.
@@ -967,28 +962,26 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
         if (e != hipSuccess) return e;
     }
     if (aux) {
-        if (t != 16) return hipErrorInvalidValue;  // depth / normal losses: 16-px tiles
-        go(launch_bwd<true, 16, 128>);
+        if (t != 16 || grad_coef.wide) return hipErrorInvalidValue;  // depth / normal losses: 16-px tiles, f32 slots
+        launch(raster_bwd_kernel<true, 16, 128, float>, static_cast<float*>(grad_coef.data), grid, 128);
     } else if (t == 8 && b == 64) {
-        go(launch_bwd<false, 8, 64>);
+        go(raster_bwd_kernel<false, 8, 64, float>, raster_bwd_kernel<false, 8, 64, double>, grid, 64);
     } else if (t == 8 && b == 128) {
-        go(launch_bwd<false, 8, 128>);
+        go(raster_bwd_kernel<false, 8, 128, float>, raster_bwd_kernel<false, 8, 128, double>, grid, 64);
     } else if (t == 16) {
         // One wave per tile: twice the workgroups for the same waves per CU.
         const uint32_t g2 = queue.cursor != nullptr ? std::min(most, std::max(2 * queue.grid_blocks, 1u))
                                                     : total_tiles;
         if (b == 64)
-            hipLaunchKernelGGL(raster_bwd_wave_kernel<64>, dim3(g2), dim3(64), 0, st, cams_dev, n_views, ranges,
-                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
+            go(raster_bwd_wave_kernel<64, float>, raster_bwd_wave_kernel<64, double>, g2, 64);
         else if (b == 128)
-            hipLaunchKernelGGL(raster_bwd_wave_kernel<128>, dim3(g2), dim3(64), 0, st, cams_dev, n_views, ranges,
-                               payloads, recs, in, grad_coef, cull, total_tiles, queue, tile_begin, sg);
+            go(raster_bwd_wave_kernel<128, float>, raster_bwd_wave_kernel<128, double>, g2, 64);
         else
             return hipErrorInvalidValue;
     } else if (t == 32 && b == 128) {
-        go(launch_bwd<false, 32, 128>);
+        go(raster_bwd_kernel<false, 32, 128, float>, raster_bwd_kernel<false, 32, 128, double>, grid, 512);
     } else if (t == 32 && b == 256) {
-        go(launch_bwd<false, 32, 256>);
+        go(raster_bwd_kernel<false, 32, 256, float>, raster_bwd_kernel<false, 32, 256, double>, grid, 512);
     } else {
         return hipErrorInvalidValue;
     }

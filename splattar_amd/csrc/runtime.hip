@@ -599,7 +599,7 @@ struct RasterCore {
     float4* out_aux = nullptr;
     float4* out_normal = nullptr;
     uint32_t* ncontrib = nullptr;
-    float* grad_coef = nullptr;
+    CoefSlots grad_coef;
     float* cam_partials = nullptr;
     BwdSegments segs;                // long lists of the backward, split over depth
     // Decision trace of the forward (verification aid; lists == nullptr: off).
@@ -658,7 +658,7 @@ struct RasterCore {
         dfree(out_aux);
         dfree(out_normal);
         dfree(ncontrib);
-        dfree(grad_coef);
+        dfree(grad_coef.data);
         dfree(cam_partials);
         dfree(segs.ctl);
         dfree(segs.table);
@@ -744,7 +744,12 @@ struct RasterCore {
         GS_CHECK(dalloc(&out_aux, pixels, "out_aux"));
         GS_CHECK(dalloc(&out_normal, pixels, "out_normal"));
         GS_CHECK(dalloc(&ncontrib, pixels, "ncontrib"));
-        GS_CHECK(dalloc(&grad_coef, nv * kGradStride, "grad_coef"));
+        // aux passes take grad_stride(true) slots, in f32.
+        const size_t slots = nv * grad_stride(aux);
+        grad_coef.wide = !aux && slots * sizeof(double) <= kWideSlotBytes;
+        uint8_t* gp = nullptr;
+        GS_CHECK(dalloc(&gp, grad_coef.bytes(slots), "grad_coef"));
+        grad_coef.data = gp;
         segs.pool = segment_pool(entries, tiles);
         GS_CHECK(dalloc(&segs.ctl, 2, "segment control"));
         GS_CHECK(dalloc(&segs.table, segs.pool, "segment table"));
@@ -2378,14 +2383,13 @@ gs_status gs_trainer_s::enqueue_step(hipStream_t st, const uint32_t* ids, uint32
             GS_HIP(launch_l1_ssim(st, tv.width, tv.height, cfg.lambda, cfg.dssim_scale, core.out_color,
                                   targets, dl_dcolor, loss_partials + (size_t)j * partials_per_view * 2,
                                   core.cams_dev + j, target_stats));
-            // Whole lists: a plain step is the form that others are compared
-            // with, and the tiles then add to a record in much the same order
-            // from run to run (gradients of the scales 2.0e-6 apart normwise,
-            // 3.2e-6 with segments, which the first Adam steps amplify for
-            // gradients near 0). 250k surfels, two 1283 x 717 views: 2.0 ms
-            // instead of 1.26 with segments.
+            // f32 slots: whole lists. A plain step leaves its gradients to the
+            // caller, and the tiles of whole lists add to a record in much the
+            // same order from run to run (250k surfels, two 1283 x 717 views:
+            // gradients of the scales 2.0e-6 apart normwise between two runs,
+            // 3.2e-6 with segments; 2.0 ms against 1.26).
             GS_CHECK(core.backward(st, j, 1, n, positions, scales, quats, sh, dl_dcolor, nullptr, g,
-                                   j > 0, false, P, true, false));
+                                   j > 0, false, P, true, core.grad_coef.wide));
         }
         if (P) GS_CHECK(P->mark(st, GS_STAGE_ADAM));
         GS_CHECK(gs_optim_encode_step(optim, st));
@@ -2413,8 +2417,8 @@ gs_status gs_trainer_s::enqueue_pipelined(hipStream_t st, const uint32_t* ids, u
     const uint32_t ka = k / 2;
     const uint32_t ta = core.cams[ka].tile_base;
     const uint32_t tt = core.total_tiles;
-    GS_HIP(launch_fill_u32(st, reinterpret_cast<uint32_t*>(core.grad_coef), 0u,
-                           (size_t)n * k * grad_stride(false)));
+    GS_HIP(launch_fill_u32(st, static_cast<uint32_t*>(core.grad_coef.data), 0u,
+                           core.grad_coef.bytes((size_t)n * k * grad_stride(false)) / sizeof(uint32_t)));
     GS_CHECK(core.raster_fwd_range(st, 0, 0, k, 0, ta));
     GS_HIP(hipEventRecord(ev[0], st));
     GS_CHECK(core.raster_fwd_range(st, 1, 0, k, ta, tt - ta));
