@@ -807,7 +807,8 @@ struct BwdSegments {
     uint32_t* ctl = nullptr;     // [0] segments in use, [1] records per segment
     uint2* table = nullptr;      // per segment: tile, index | kSegmentLast (tile ~0: none)
     uint32_t* split = nullptr;   // per tile: 1 = walked by segments
-    float4* state = nullptr;     // [1, with aux 3][pool][kSegmentPixels]
+    float4* state = nullptr;      // [pool][kSegmentPixels]
+    float4* state_aux = nullptr;  // [2][pool][kSegmentPixels], for passes with aux
     uint32_t pool = 0;
 };
 // A segment holds L records, L a multiple of 32 of at least E / kSegmentTarget

@@ -228,25 +228,23 @@ __device__ __forceinline__ void step_state(PixState& p, const Record& r, const H
 // tile (8x8 block k >> 6, row-major within it) of segment `at`.
 template <bool AUX>
 __device__ __forceinline__ void store_state(const BwdSegments& sg, uint32_t at, uint32_t k, const PixState& p) {
-    float4* dst = sg.state + (size_t)at * kSegmentPixels + k;
-    const size_t plane = (size_t)sg.pool * kSegmentPixels;
-    dst[0] = make_float4(p.T, p.suf_r, p.suf_g, p.suf_b);
+    const size_t j = (size_t)at * kSegmentPixels + k;
+    sg.state[j] = make_float4(p.T, p.suf_r, p.suf_g, p.suf_b);
     if (AUX) {
-        dst[plane] = make_float4(p.suf_d, p.suf_nx, p.suf_ny, p.suf_nz);
-        dst[2 * plane] = make_float4(p.suf_w, p.suf_cw, 0.0f, 0.0f);
+        sg.state_aux[j] = make_float4(p.suf_d, p.suf_nx, p.suf_ny, p.suf_nz);
+        sg.state_aux[(size_t)sg.pool * kSegmentPixels + j] = make_float4(p.suf_w, p.suf_cw, 0.0f, 0.0f);
     }
 }
 template <bool AUX>
 __device__ __forceinline__ void load_state(const BwdSegments& sg, uint32_t at, uint32_t k, PixState& p) {
-    const float4* src = sg.state + (size_t)at * kSegmentPixels + k;
-    const size_t plane = (size_t)sg.pool * kSegmentPixels;
-    const float4 a = src[0];
+    const size_t j = (size_t)at * kSegmentPixels + k;
+    const float4 a = sg.state[j];
     p.T = a.x;
     p.suf_r = a.y;
     p.suf_g = a.z;
     p.suf_b = a.w;
     if (AUX) {
-        const float4 b = src[plane], c = src[2 * plane];
+        const float4 b = sg.state_aux[j], c = sg.state_aux[(size_t)sg.pool * kSegmentPixels + j];
         p.suf_d = b.x;
         p.suf_nx = b.y;
         p.suf_ny = b.z;
@@ -830,7 +828,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStateWaves
         if (tid == 0) s_base = atomicAdd(sg.ctl, nseg);
         __syncthreads();
         const uint32_t at = __builtin_amdgcn_readfirstlane(s_base);
-        const bool room = at + nseg <= sg.pool;  // by segment_pool always
+        const bool room = at + nseg <= sg.pool;  // always, unless the pool was capped
         for (uint32_t k = (uint32_t)tid; k < nseg && at + k < sg.pool; k += 256)
             sg.table[at + k] = make_uint2(room ? gtile : ~0u, k + 1 == nseg ? k | kSegmentLast : k);
         if (tid == 0 && room) sg.split[gtile] = 1u;

@@ -601,7 +601,7 @@ struct RasterCore {
     uint32_t* ncontrib = nullptr;
     CoefSlots grad_coef;
     float* cam_partials = nullptr;
-    BwdSegments segs;                // long lists of the backward, split over depth
+    BwdSegments segs;                // long lists of the backward, split over depth (segments())
     // Decision trace of the forward (verification aid; lists == nullptr: off).
     FwdTrace trace;
     // Depth-presort path (binning = GS_BINNING_PRESORT or GS_BINNING_TIGHT).
@@ -664,6 +664,7 @@ struct RasterCore {
         dfree(segs.table);
         dfree(segs.split);
         dfree(segs.state);
+        dfree(segs.state_aux);
         for (int i = 0; i < 2; ++i) {
             dfree(pre_keys[i]);
             dfree(pre_vals[i]);
@@ -679,8 +680,7 @@ struct RasterCore {
         dfree(cursors);
     }
 
-    // aux: backward passes with depth / normal losses may run (their segment
-    // states hold three vectors per pixel instead of one).
+    // aux: backward passes with depth / normal losses may run.
     gs_status init(gs_ctx c, uint32_t n, uint32_t views, uint32_t entries, uint32_t tiles,
                    uint32_t pixels, bool aux) {
         ctx = c;
@@ -751,11 +751,11 @@ struct RasterCore {
         GS_CHECK(dalloc(&gp, grad_coef.bytes(slots), "grad_coef"));
         grad_coef.data = gp;
         segs.pool = segment_pool(entries, tiles);
+        // GS_SEGMENT_POOL caps it (a tile without room is walked whole).
+        if (const char* env = std::getenv("GS_SEGMENT_POOL"))
+            segs.pool = std::min(segs.pool, (uint32_t)std::max(std::atoi(env), 1));
         GS_CHECK(dalloc(&segs.ctl, 2, "segment control"));
-        GS_CHECK(dalloc(&segs.table, segs.pool, "segment table"));
         GS_CHECK(dalloc(&segs.split, tiles, "split tiles"));
-        GS_CHECK(dalloc(&segs.state, (size_t)segs.pool * kSegmentPixels * (aux ? 3 : 1), "segment states",
-                        false));
         uint8_t* cp = nullptr;
         GS_CHECK(dalloc(&cp, geom_cam_partials_bytes(n, views), "camera partials"));
         cam_partials = reinterpret_cast<float*>(cp);
@@ -963,6 +963,25 @@ struct RasterCore {
         return GS_OK;
     }
 
+    // The segment buffers a backward pass needs, allocated by the first that
+    // splits lists (27 to 52 MB, with aux three times that: not for a rasterizer
+    // that only renders) and kept until the object goes, since a captured pass
+    // holds their addresses. That first pass may itself be under capture, on
+    // this thread or another: an allocation is no part of it, so it is made in
+    // relaxed mode.
+    gs_status segments(bool aux) {
+        if (segs.state != nullptr && (!aux || segs.state_aux != nullptr)) return GS_OK;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        GS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        const size_t plane = (size_t)segs.pool * kSegmentPixels;
+        gs_status s = GS_OK;
+        if (segs.table == nullptr) s = dalloc(&segs.table, segs.pool, "segment table", false);
+        if (s == GS_OK && aux && segs.state_aux == nullptr) s = dalloc(&segs.state_aux, 2 * plane, "segment states", false);
+        if (s == GS_OK && segs.state == nullptr) s = dalloc(&segs.state, plane, "segment states", false);
+        GS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        return s;
+    }
+
     gs_status backward(hipStream_t st, uint32_t v0, uint32_t nv, uint32_t n, const float4* pos,
                        const float2* sc, const float4* q, const float* sh, const float4* dl_dcolor,
                        const float4* dl_dnormal, ParamGrads g, bool accumulate, bool aux,
@@ -975,6 +994,9 @@ struct RasterCore {
         GS_CHECK(P.mark(st, GS_STAGE_GRAD_CLEAR));
         BwdIn in{dl_dcolor, dl_dnormal, out_color, out_aux, ncontrib};
         const TileQueue qb = (q_tiles[0] == tiles && q_begin[0] == 0) ? queue(0, 1) : TileQueue{nullptr, nullptr, 0};
+        // Segments need the queue (its order and cursors) and 16-px tiles.
+        split = split && qb.cursor != nullptr && shape.tile == (uint32_t)kTile;
+        if (split) GS_CHECK(segments(aux));
         GS_HIP(launch_bwd_prepare(st, grad_coef, (size_t)n * nv * grad_stride(aux), qb.cursor, segs, tiles,
                                   last_sort_count, aux));
         GS_CHECK(P.mark(st, GS_STAGE_RASTER_BWD));
@@ -2487,6 +2509,9 @@ gs_status gs_trainer_create(gs_ctx ctx, const gs_train_config* cfg, const gs_sce
         const char* env = std::getenv("GS_PIPELINE");
         t->pipeline = env != nullptr && env[0] == '1';
     }
+    // Its steps split lists, unless they are overlapped or without the queue:
+    // the buffers now rather than in the first step (1.3 ms instead of 0.32).
+    if (t->core.tile_queue && !t->pipeline) GS_CHECK(t->core.segments(false));
     GS_CHECK(dalloc(&t->targets, toff, "targets"));
     {
         std::vector<float> buf;
