@@ -393,8 +393,7 @@ __device__ __forceinline__ uint32_t small_rounds(uint32_t n) { return (n + kSmal
 template <typename K, int RB>
 __device__ __forceinline__ uint32_t small_sort(K (&key)[kSmallItems], uint32_t (&val)[kSmallItems], uint32_t n,
                                                uint32_t begin_bit, uint32_t passes, bool drop,
-                                               K* __restrict__ kout, uint32_t* __restrict__ vout,
-                                               SmallShared<K, RB>& sm) {
+                                               K* kout, uint32_t* vout, SmallShared<K, RB>& sm) {
     constexpr uint32_t R = 1u << RB;
     constexpr int ITEMS = kSmallItems;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -471,9 +470,10 @@ __device__ __forceinline__ uint32_t small_sort(K (&key)[kSmallItems], uint32_t (
     return n;
 }
 
+// After an even number of passes the output is the input's buffers: no
+// __restrict__. Every pair is read before the first barrier.
 template <typename K, int RB>
-__global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(const K* __restrict__ kin,
-                                                                   const uint32_t* __restrict__ vin, K* kout,
+__global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(const K* kin, const uint32_t* vin, K* kout,
                                                                    uint32_t* vout,
                                                                    const uint32_t* __restrict__ count, uint32_t cap,
                                                                    uint32_t begin_bit, uint32_t passes,
