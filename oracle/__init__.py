@@ -771,3 +771,26 @@ def xorshift32(seed: int, n: int, modulus: int = 0) -> np.ndarray:
 
 def num_threads() -> int:
     return int(lib().oref_num_threads())
+
+
+# ---------------------------------------------------------- footprint replay
+
+FOOTPRINT_TESTS = ("tile 16", "block 8x8 of 16", "sub-block 4x4 of 16", "tile 8", "block of 8", "sub-block of 8",
+                   "tile 32", "block 8x8 of 32")
+
+
+def footprint_replay(seed: int, n: int, width: int, height: int, kind: int) -> dict:
+    """The product's footprint tests over every pixel of n random records
+    (footprint_replay.cpp): accepted evaluations, those each test left out,
+    the share of 4x4 tests that keep a record, records with a bounded ellipse,
+    and the largest relative error of a stored disk radius."""
+    fn = lib().oref_footprint_replay
+    fn.argtypes = [C.c_uint64, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int, C.POINTER(C.c_uint64),
+                   C.POINTER(C.c_double)]
+    fn.restype = C.c_int
+    out, err = (C.c_uint64 * 16)(), C.c_double()
+    if fn(seed, n, width, height, kind, out, C.byref(err)) != 0:
+        raise ValueError("footprint_replay: bad arguments")
+    return {"hits": int(out[0]), "misses": dict(zip(FOOTPRINT_TESTS, (int(v) for v in out[1:9]))),
+            "kept": out[9] / max(out[10], 1), "bounded": int(out[11]), "records": int(out[12]),
+            "radius_err": err.value}
