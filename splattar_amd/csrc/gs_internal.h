@@ -857,10 +857,11 @@ hipError_t launch_geom_bwd(hipStream_t st, const CamParams* cams_dev, uint32_t n
 // per-view descriptor lives in device memory, so a captured graph replays
 // with whatever views the descriptor table holds). partial_sums, room for
 // l1_ssim_partials(w, h) pairs, receives the number of sums and as many pairs
-// (sum |x - y|, sum SSIM) after that pair; dl_out may be null (loss only). tstats, when set, holds the target's window mean and second
-// moment per channel (launch_target_stats), at (target pixel) * 3 + channel
-// from the same base offset as the target.
-hipError_t launch_l1_ssim(hipStream_t st, uint32_t w, uint32_t h, float lambda, float dssim_scale,
+// (sum |x - y|, sum SSIM) after that pair; dl_out may be null (loss only).
+// tstats, when set, holds the target's window mean and second moment per
+// channel (launch_target_stats), at (target pixel) * 3 + channel from the same
+// base offset as the target. cus: the device's compute units.
+hipError_t launch_l1_ssim(hipStream_t st, uint32_t cus, uint32_t w, uint32_t h, float lambda, float dssim_scale,
                           const float4* img, const float4* target, float4* dl_out, double* partial_sums,
                           const CamParams* view = nullptr, const float2* tstats = nullptr);
 uint32_t l1_ssim_partials(uint32_t w, uint32_t h);
@@ -872,7 +873,7 @@ hipError_t launch_target_stats(hipStream_t st, uint32_t w, uint32_t h, const flo
 // j's image and dL/dimage start at img / dl_out + pix_base[j], its target at
 // target + cams_dev[first + j].target_base, its partial sums at
 // partials + 2 (first + j) partials_stride. At most 64 views.
-hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t first, uint32_t k, const uint32_t* widths,
+hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t cus, uint32_t first, uint32_t k, const uint32_t* widths,
                                 const uint32_t* heights, const uint32_t* pix_base, float lambda,
                                 float dssim_scale, const float4* img, const float4* target, float4* dl_out,
                                 double* partials, uint32_t partials_stride, const CamParams* cams_dev,

@@ -339,16 +339,15 @@ constexpr uint32_t kMinRows = 4;
 // Rows per band. A band of r rows works through r + 21 steps, the first 20 of
 // them short, so longer bands do less work; but the steps are serial, 1.1 us
 // each for a workgroup alone on its CU, and it takes four a CU to fill it
-// (1.95 us a step). Measured for c workgroups a CU (256 CUs): kStep[c] r +
+// (1.95 us a step). Measured for c workgroups a CU (256 of them): kStep[c] r +
 // kStart[c] us; more than four a CU run in rounds of four. The shortest
 // estimate is taken (a longer band where two agree). Against 64 rows always:
 // 256 x 256 89 -> 23 us, 1080p 104 -> 77 us, 1283 x 717 95 -> 52 us, eight
 // uneven views 382 -> 333 us, four 1080p 268 -> 249 us, sixteen 720p 483 ->
 // 428 us. dL/dimage does not depend on the bands; the double sums are grouped
 // by band, so a view's loss may differ in its last bits between launches.
-uint32_t band_rows(const LossViews& lv) {
+uint32_t band_rows(const LossViews& lv, uint32_t cus) {
     constexpr float kStep[5] = {0.f, 1.1f, 1.3f, 1.65f, 1.95f}, kStart[5] = {0.f, 18.f, 22.f, 22.f, 22.f};
-    constexpr uint32_t kCus = 256;
     uint32_t max_h = 0, best = kMinRows, strips[kMaxLossViews];
     for (uint32_t j = 0; j < lv.n; ++j) {
         max_h = std::max(max_h, lv.h[j]);
@@ -359,7 +358,7 @@ uint32_t band_rows(const LossViews& lv) {
         const uint32_t bands = div_up(max_h, r), rows = std::max(kMinRows, div_up(max_h, bands));
         uint64_t blocks = 0;
         for (uint32_t j = 0; j < lv.n; ++j) blocks += (uint64_t)strips[j] * div_up(lv.h[j], rows);
-        const uint64_t rounds = blocks / (4 * kCus), c = div_up(blocks % (4 * kCus), (uint64_t)kCus);
+        const uint64_t rounds = blocks / (4 * cus), c = div_up(blocks % (4 * cus), cus);
         const float us = (float)rounds * (kStep[4] * (float)rows + kStart[4]) + kStep[c] * (float)rows + kStart[c];
         if (us <= best_us) {
             best_us = us;
@@ -369,9 +368,9 @@ uint32_t band_rows(const LossViews& lv) {
     }
 }
 
-hipError_t launch_fused(hipStream_t st, LossViews& lv, const float4* img, const float4* target, float4* dl_out,
+hipError_t launch_fused(hipStream_t st, uint32_t cus, LossViews& lv, const float4* img, const float4* target, float4* dl_out,
                         double* partials, const CamParams* cams, const float2* tstats) {
-    lv.rows = band_rows(lv);
+    lv.rows = band_rows(lv, cus);
     uint32_t blocks = 0;
     for (uint32_t j = 0; j < lv.n; ++j) {
         lv.block_begin[j] = blocks;
@@ -442,7 +441,7 @@ hipError_t launch_target_stats(hipStream_t st, uint32_t w, uint32_t h, const flo
     return hipGetLastError();
 }
 
-hipError_t launch_l1_ssim(hipStream_t st, uint32_t w, uint32_t h, float lambda, float dssim_scale,
+hipError_t launch_l1_ssim(hipStream_t st, uint32_t cus, uint32_t w, uint32_t h, float lambda, float dssim_scale,
                           const float4* img, const float4* target, float4* dl_out, double* partial_sums,
                           const CamParams* view, const float2* tstats) {
     if (w == 0 || h == 0) return hipSuccess;
@@ -451,10 +450,10 @@ hipError_t launch_l1_ssim(hipStream_t st, uint32_t w, uint32_t h, float lambda, 
     lv.w[0] = w;
     lv.h[0] = h;
     loss_weights(w, h, lambda, dssim_scale, &lv.dw[0], &lv.l1w[0]);
-    return launch_fused(st, lv, img, target, dl_out, partial_sums, view, tstats);
+    return launch_fused(st, cus, lv, img, target, dl_out, partial_sums, view, tstats);
 }
 
-hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t first, uint32_t k, const uint32_t* widths,
+hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t cus, uint32_t first, uint32_t k, const uint32_t* widths,
                                 const uint32_t* heights, const uint32_t* pix_base, float lambda,
                                 float dssim_scale, const float4* img, const float4* target, float4* dl_out,
                                 double* partials, uint32_t partials_stride, const CamParams* cams_dev,
@@ -471,7 +470,7 @@ hipError_t launch_l1_ssim_views(hipStream_t st, uint32_t first, uint32_t k, cons
         lv.pix_base[j] = pix_base[j];
         loss_weights(widths[j], heights[j], lambda, dssim_scale, &lv.dw[j], &lv.l1w[j]);
     }
-    return launch_fused(st, lv, img, target, dl_out, partials, cams_dev, tstats);
+    return launch_fused(st, cus, lv, img, target, dl_out, partials, cams_dev, tstats);
 }
 
 }  // namespace gs

@@ -148,6 +148,8 @@ struct gs_context {
     uint32_t* noalloc_scratch = nullptr;
 };
 
+static uint32_t compute_units(gs_ctx ctx) { return (uint32_t)std::max(1, ctx->props.multiProcessorCount); }
+
 namespace gs {
 
 // Scratch of gs_scan_encode_noalloc: the partition sums of a scan of up to
@@ -729,7 +731,7 @@ struct RasterCore {
             // selects one workgroup per tile in tile order instead.
             const char* env = std::getenv("GS_TILE_QUEUE");
             tile_queue = !(env != nullptr && env[0] == '0');
-            cus = (uint32_t)std::max(1, ctx->props.multiProcessorCount);
+            cus = compute_units(ctx);
             queue_blocks = 8u * cus;
         }
         for (int i = 0; i < 2; ++i) {
@@ -1379,7 +1381,7 @@ gs_status gs_loss_set_dssim_scale(gs_loss l, float scale) {
 
 gs_status gs_loss_encode(gs_loss l, void* stream) {
     GS_REQUIRE(l != nullptr, "loss is null");
-    GS_HIP(launch_l1_ssim(as_stream(stream, l->ctx->stream), l->width, l->height, l->lambda,
+    GS_HIP(launch_l1_ssim(as_stream(stream, l->ctx->stream), compute_units(l->ctx), l->width, l->height, l->lambda,
                           l->dssim_scale, l->img, l->target, l->dl_out, l->partials));
     return GS_OK;
 }
@@ -2308,7 +2310,7 @@ struct gs_trainer_s {
     gs_status loss_view(hipStream_t s, const uint32_t* ids, uint32_t j) {
         const TrainViewDev& tv = views[ids[j]];
         const CamParams& c = core.cams[j];
-        GS_HIP(launch_l1_ssim(s, tv.width, tv.height, cfg.lambda, cfg.dssim_scale, core.out_color + c.pix_base,
+        GS_HIP(launch_l1_ssim(s, core.cus, tv.width, tv.height, cfg.lambda, cfg.dssim_scale, core.out_color + c.pix_base,
                               targets, dl_dcolor + c.pix_base,
                               loss_partials + (size_t)j * partials_per_view * 2, core.cams_dev + j,
                               target_stats));
@@ -2329,7 +2331,7 @@ struct gs_trainer_s {
             hs[j] = tv.height;
             pb[j] = core.cams[j0 + j].pix_base;
         }
-        GS_HIP(launch_l1_ssim_views(s, j0, k, ws.data(), hs.data(), pb.data(), cfg.lambda, cfg.dssim_scale,
+        GS_HIP(launch_l1_ssim_views(s, core.cus, j0, k, ws.data(), hs.data(), pb.data(), cfg.lambda, cfg.dssim_scale,
                                     core.out_color, targets, dl_dcolor, loss_partials, partials_per_view,
                                     core.cams_dev, target_stats));
         return GS_OK;
@@ -2402,7 +2404,7 @@ gs_status gs_trainer_s::enqueue_step(hipStream_t st, const uint32_t* ids, uint32
             const TrainViewDev& tv = views[ids[j]];
             GS_CHECK(core.forward(st, j, 1, n, positions, scales, quats, opacities, sh, P));
             if (P) GS_CHECK(P->mark(st, GS_STAGE_LOSS));
-            GS_HIP(launch_l1_ssim(st, tv.width, tv.height, cfg.lambda, cfg.dssim_scale, core.out_color,
+            GS_HIP(launch_l1_ssim(st, core.cus, tv.width, tv.height, cfg.lambda, cfg.dssim_scale, core.out_color,
                                   targets, dl_dcolor, loss_partials + (size_t)j * partials_per_view * 2,
                                   core.cams_dev + j, target_stats));
             // f32 slots: whole lists. A plain step leaves its gradients to the
@@ -2688,7 +2690,7 @@ gs_status gs_trainer_set_schedule(gs_trainer t, uint32_t digit_bits, uint32_t bl
     GS_REQUIRE(t != nullptr, "trainer is null");
     GS_REQUIRE(digit_bits == 4 || digit_bits == 8, "digit_bits must be 4 or 8");
     GS_REQUIRE(blocks_per_cu <= 64, "blocks_per_cu must be <= 64");
-    const uint32_t cus = (uint32_t)std::max(1, t->ctx->props.multiProcessorCount);
+    const uint32_t cus = compute_units(t->ctx);
     t->core.digit_bits = digit_bits;
     t->core.tile_queue = blocks_per_cu != 0;
     t->core.queue_blocks = std::max(1u, blocks_per_cu) * cus;
@@ -2838,7 +2840,7 @@ gs_status gs_trainer_autotune(gs_trainer t, const uint32_t* view_ids, uint32_t n
     if (s == GS_OK) s = rs;
     if (s != GS_OK || b1 >= cands.size() || b2 >= stage2.size()) {
         // Failure, or every candidate overflowed: back to the schedule on entry.
-        const uint32_t cus = (uint32_t)std::max(1, t->ctx->props.multiProcessorCount);
+        const uint32_t cus = compute_units(t->ctx);
         (void)gs_trainer_set_schedule(t, digit0, queue0 / cus);
         (void)gs_trainer_set_tiling(t, shape0.tile, shape0.fwd_batch, shape0.bwd_batch);
         GS_CHECK(s);
