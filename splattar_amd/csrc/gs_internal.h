@@ -815,11 +815,11 @@ struct BwdSegments {
 // rounded down (E = entries), so all lists together have at most E / L <= 33/32
 // kSegmentTarget whole segments and each split tile, longer than L, one more;
 // there are no more split tiles than E / L either.
-// Measured at 6144 and 32 against
-// half and twice the target (250k 2x1283x717 1738 against 1827 / 1732 us),
-// batch 200k 6x640x360 1857 against 1965 / 1815 us, 100k eight uneven views 1557
-// against 1558 / 1642 us; a minimum of 64 loses 3 % at 10k 256px (396 against
-// 384 us) and gains 9 % with aux (20k 321x243: 483 against 531 us).
+// Measured at 6144 and 32 against half and twice the target, a step or pass:
+// 250k surfels in two 1283 x 717 views (batched) 945 us against 1025 / 944, 200k
+// in six 640 x 360 views 1433 against 1559 / 1418, 100k in eight uneven views
+// 1428 against 1381 / 1605; a minimum of 64 loses 6 % at 10k 256 x 256 (232
+// against 219 us) and gains 3 % with aux (20k 321 x 243: 307 against 318).
 constexpr uint32_t segment_pool(uint32_t max_entries, uint32_t tiles) {
     constexpr uint64_t whole = kSegmentTarget + kSegmentTarget / 32 + 1;
     const uint64_t by_entries = 2ull * max_entries / kSegmentMin, by_tiles = whole + (tiles < whole ? tiles : whole);

@@ -17,10 +17,10 @@
 //     gradient with hardware global atomics, FP32 or FP64 (no CAS loops). A 32x32
 //     tile is eight waves, each owning an 8-wide, 16-tall column of two
 //     blocks (two pixels per lane), whose per-record reductions meet in LDS
-//     slots (ds_add_f32) flushed once per batch (the two waves of the depth /
-//     normal variant each have a copy of them); an 8x8 tile is one wave with
-//     one pixel per lane (raster_bwd_kernel). Records are staged BATCH at a
-//     time into order-preserving lists that carry the blocks each reaches;
+//     slots (ds_add_f32) flushed once per batch, as do those of the two waves of
+//     the depth / normal variant; an 8x8 tile is one wave with one pixel per
+//     lane (raster_bwd_kernel). Records are staged BATCH at a time into
+//     order-preserving lists that carry the blocks each reaches;
 //   * each wave reduces its lanes' 16 values with a transposed butterfly (17
 //     lane exchanges instead of 96, on permlane swaps and DPP rather than LDS
 //     permutes);
@@ -361,8 +361,15 @@ __device__ __forceinline__ void add_hit(PixState& p, const Record& r, const HitE
     }
 }
 
+// Waves per SIMD: with depth and normals three (168 registers), where the
+// compiler's 174 leave two: a backward pass of 1M surfels at 1080p 1845 -> 1604
+// us, 300k at 720p 877 -> 744, 20k at 321 x 243 160 -> 155; with no more
+// workgroups than then fit (launch_raster_bwd) 1490, 739 and 153. A copy of the
+// slots per wave instead of LDS adds takes 10 KB more, so five workgroups a CU
+// instead of six: 1607, 791 and 155.
 template <bool AUX, int TW, int BATCH, typename Slot>
-__global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
+__global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2)
+__attribute__((amdgpu_waves_per_eu(AUX ? 3 : 1))) void raster_bwd_kernel(
     const CamParams* __restrict__ cams, uint32_t n_views, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ payloads, const Record* __restrict__ recs, BwdIn in,
     Slot* __restrict__ grad_coef, bool cull, uint32_t total_tiles, TileQueue queue, uint32_t tile_begin,
@@ -381,11 +388,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
     __shared__ uint16_t s_list[NW][BATCH + 1];  // read one entry ahead
     __shared__ uint32_t s_wlast[NW][2];        // last contributors of each wave's blocks
     __shared__ uint32_t s_qcnt[SW][NW];      // [staging wave][list wave]
-    // One or two waves: a copy of the slots per wave, written (a wave meets a
-    // record once per batch) and summed at the flush; LDS float atomics run at
-    // one lane per ~3 cycles. Eight waves (32-px tiles) share one copy.
-    constexpr int NG = NW <= 2 ? NW : 1;
-    __shared__ float s_grad[NG][BATCH * NS];
+    __shared__ float s_grad[BATCH * NS];
     __shared__ uint32_t s_view, s_maxlast, s_next;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -490,10 +493,7 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                     if (lane == 0) s_qcnt[sw][w] = (uint32_t)__popcll(bal);
                 }
             }
-            for (int k = tid; k < (int)cnt * NS; k += NT) {
-#pragma unroll
-                for (int c = 0; c < NG; ++c) s_grad[c][k] = 0.0f;
-            }
+            for (int k = tid; k < (int)cnt * NS; k += NT) s_grad[k] = 0.0f;
             __syncthreads();
 #pragma unroll
             for (int m = 0; m < SPT; ++m) {
@@ -562,20 +562,19 @@ __global__ __launch_bounds__(TW == 8 ? 64 : TW * TW / 2) void raster_bwd_kernel(
                 }
                 const float red = wave_sums16(g);
                 if ((lane & 3) == 0) {
-                    float* const dst = &s_grad[NG > 1 ? wave : 0][j * NS + (lane >> 2)];
-                    if constexpr (NG == NW) *dst = red;
+                    // One wave meets a record once per batch: no other adds.
+                    float* const dst = &s_grad[j * NS + (lane >> 2)];
+                    if constexpr (NW == 1) *dst = red;
                     else if (red != 0.0f) atomicAdd(dst, red);
                 }
                 if (AUX) {
-                    static_assert(!AUX || NG == NW, "a copy of the slots per wave");
                     const float red2 = wave_sums4(g2);
-                    if ((lane & 15) == 0) s_grad[NG > 1 ? wave : 0][j * NS + 16 + (lane >> 4)] = red2;
+                    if ((lane & 15) == 0 && red2 != 0.0f) atomicAdd(&s_grad[j * NS + 16 + (lane >> 4)], red2);
                 }
             }
             __syncthreads();
             for (int k = tid; k < (int)cnt * NS; k += NT) {
-                float v = s_grad[0][k];
-                if constexpr (NG == 2) v += s_grad[1][k];
+                const float v = s_grad[k];
                 if (v != 0.0f) {
                     const int e = k / NS, slot = k - e * NS;
                     // A colour channel clamped at 0 in the forward passes no
@@ -762,15 +761,15 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(float4* __restrict__ g
 // pixels here, so each 16-lane row walks its own list of the records that
 // reach its 4x4 sub-block: a list is about a third of the tile's, and a
 // record's step has 45 instructions against ~230 with gradients and their
-// reduction, which is what shortens the critical path. 250k surfels at 1283 x
-// 717: 83 us for the state pass and 190 us for the gradient pass, where a
-// gradient pass over whole lists took 1042 us (its longest list); 200k surfels
-// in six 640 x 360 views: 220 + 610 against 2085 us. Where no list is longer
-// than a segment (1M surfels, four 1080p views) the pass is 10 us.
+// reduction, which is what shortens the critical path. 250k surfels in two 1283
+// x 717 views: 100 us for the state pass and 375 for the gradient pass, where a
+// gradient pass over whole lists takes 679 us (its longest list); 200k surfels
+// in six 640 x 360 views: 219 + 609 against 1373 us. Where no list is longer
+// than a segment the pass is 10 us.
 // Batches of 256 records that do not stop at segment boundaries, staged one
 // record a thread: 281 -> 220 us for the six views, 105 -> 71 us with aux (20k
-// surfels at 321 x 243), 92 -> 83 us for the 1283 x 717 one, against batches of
-// a segment (at most 128, two threads a record).
+// surfels at 321 x 243), against batches of a segment (at most 128, two threads
+// a record).
 // Waves per SIMD: 220 us for the six views above at five, 235 at four, 295 at
 // six (19 spilled registers); with aux 71 us at four, 84 at five.
 template <bool AUX>
@@ -913,6 +912,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStateWaves
     }
 }
 
+// Workgroups of a kernel that a CU holds.
+template <auto Kernel>
+uint32_t resident(uint32_t threads) {
+    static const uint32_t fit = [threads] {
+        int n = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, Kernel, (int)threads, 0);
+        return e == hipSuccess && n > 0 ? (uint32_t)n : 1u;
+    }();
+    return fit;
+}
+
 }  // namespace
 
 hipError_t launch_bwd_prepare(hipStream_t st, CoefSlots grad_coef, size_t slots, uint32_t* cursor, BwdSegments sg,
@@ -937,14 +947,21 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
     // Segments need the queue (its order and cursors) and 16-px tiles.
     if (queue.cursor == nullptr || t != 16) sg = BwdSegments{};
     const uint32_t most = total_tiles + (sg.state != nullptr ? sg.pool : 0u);
-    const uint32_t grid = queue.cursor != nullptr ? std::min(most, std::max(queue.grid_blocks, 1u)) : total_tiles;
-    auto launch = [&](auto* kernel, auto* slots, uint32_t blocks, uint32_t threads) {
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, st, cams_dev, n_views, ranges, payloads, recs, in,
+    // With a queue, at most `times` workgroups for each that the schedule asks
+    // for, and no more than the CUs hold (`fit`): positions below the grid size
+    // belong to workgroups that should start at once.
+    auto launch = [&](auto* kernel, auto* slots, uint32_t threads, uint32_t fit, uint32_t times) {
+        uint32_t grid = total_tiles;
+        if (queue.cursor != nullptr) {
+            grid = std::min(most, std::max(times * queue.grid_blocks, 1u));
+            if (queue.cus != 0) grid = std::min(grid, fit * queue.cus);
+        }
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, st, cams_dev, n_views, ranges, payloads, recs, in,
                            slots, cull, total_tiles, queue, tile_begin, sg);
     };
-    auto go = [&](auto* narrow, auto* wide, uint32_t blocks, uint32_t threads) {
-        if (grad_coef.wide) launch(wide, static_cast<double*>(grad_coef.data), blocks, threads);
-        else launch(narrow, static_cast<float*>(grad_coef.data), blocks, threads);
+    auto go = [&](auto* narrow, auto* wide, uint32_t threads, uint32_t fit, uint32_t times = 1) {
+        if (grad_coef.wide) launch(wide, static_cast<double*>(grad_coef.data), threads, fit, times);
+        else launch(narrow, static_cast<float*>(grad_coef.data), threads, fit, times);
     };
     if (sg.state != nullptr) {
         // As many workgroups (four waves) as the CUs hold.
@@ -961,25 +978,27 @@ hipError_t launch_raster_bwd(hipStream_t st, const CamParams* cams_dev, const Ca
     }
     if (aux) {
         if (t != 16 || grad_coef.wide) return hipErrorInvalidValue;  // depth / normal losses: 16-px tiles, f32 slots
-        launch(raster_bwd_kernel<true, 16, 128, float>, static_cast<float*>(grad_coef.data), grid, 128);
+        launch(raster_bwd_kernel<true, 16, 128, float>, static_cast<float*>(grad_coef.data), 128,
+               resident<raster_bwd_kernel<true, 16, 128, float>>(128), 1);
     } else if (t == 8 && b == 64) {
-        go(raster_bwd_kernel<false, 8, 64, float>, raster_bwd_kernel<false, 8, 64, double>, grid, 64);
+        go(raster_bwd_kernel<false, 8, 64, float>, raster_bwd_kernel<false, 8, 64, double>, 64,
+           resident<raster_bwd_kernel<false, 8, 64, float>>(64));
     } else if (t == 8 && b == 128) {
-        go(raster_bwd_kernel<false, 8, 128, float>, raster_bwd_kernel<false, 8, 128, double>, grid, 64);
-    } else if (t == 16) {
+        go(raster_bwd_kernel<false, 8, 128, float>, raster_bwd_kernel<false, 8, 128, double>, 64,
+           resident<raster_bwd_kernel<false, 8, 128, float>>(64));
+    } else if (t == 16 && b == 64) {
         // One wave per tile: twice the workgroups for the same waves per CU.
-        const uint32_t g2 = queue.cursor != nullptr ? std::min(most, std::max(2 * queue.grid_blocks, 1u))
-                                                    : total_tiles;
-        if (b == 64)
-            go(raster_bwd_wave_kernel<64, float>, raster_bwd_wave_kernel<64, double>, g2, 64);
-        else if (b == 128)
-            go(raster_bwd_wave_kernel<128, float>, raster_bwd_wave_kernel<128, double>, g2, 64);
-        else
-            return hipErrorInvalidValue;
+        go(raster_bwd_wave_kernel<64, float>, raster_bwd_wave_kernel<64, double>, 64,
+           resident<raster_bwd_wave_kernel<64, float>>(64), 2);
+    } else if (t == 16 && b == 128) {
+        go(raster_bwd_wave_kernel<128, float>, raster_bwd_wave_kernel<128, double>, 64,
+           resident<raster_bwd_wave_kernel<128, float>>(64), 2);
     } else if (t == 32 && b == 128) {
-        go(raster_bwd_kernel<false, 32, 128, float>, raster_bwd_kernel<false, 32, 128, double>, grid, 512);
+        go(raster_bwd_kernel<false, 32, 128, float>, raster_bwd_kernel<false, 32, 128, double>, 512,
+           resident<raster_bwd_kernel<false, 32, 128, float>>(512));
     } else if (t == 32 && b == 256) {
-        go(raster_bwd_kernel<false, 32, 256, float>, raster_bwd_kernel<false, 32, 256, double>, grid, 512);
+        go(raster_bwd_kernel<false, 32, 256, float>, raster_bwd_kernel<false, 32, 256, double>, 512,
+           resident<raster_bwd_kernel<false, 32, 256, float>>(512));
     } else {
         return hipErrorInvalidValue;
     }
