@@ -213,7 +213,7 @@ struct DownsweepShared {
     uint32_t wave_hist[kSortWaves][1 << RB];   // running counts, then wave-exclusive
     uint32_t digit_start[1 << RB];             // block-local exclusive digit starts
     uint32_t out_base[1 << RB];                // global dest = out_base[d] + local pos
-    uint32_t tmp[kSortWaves];
+    uint32_t tmp[2][kSortWaves];
     uint32_t valid;                            // keys of the partition that are kept
     K buf[kSortThreads * kMaxItems];           // the keys in digit order, then the payloads
 };
@@ -269,8 +269,28 @@ __device__ __forceinline__ void downsweep_part(const K* __restrict__ kin, const 
         }
         block_count = run;
     }
-    const uint32_t digit_start = block_exclusive_scan_digits<R>(block_count, sm.tmp);
-    const uint32_t global_start = block_exclusive_scan_digits<R>(hist_d, sm.tmp);
+    // Exclusive scans of the block's counts and of the digit totals, together:
+    // one barrier for both instead of four (1M pairs 79.0 -> 76.5 us for four
+    // passes, 4M 146 -> 143, 64-bit 2M 214 -> 210 for eight).
+    uint32_t digit_start = block_count, global_start = hist_d;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t a = __shfl_up(digit_start, o), b = __shfl_up(global_start, o);
+        if (lane >= o) {
+            digit_start += a;
+            global_start += b;
+        }
+    }
+    if (lane == 63) {
+        sm.tmp[0][wave] = digit_start;
+        sm.tmp[1][wave] = global_start;
+    }
+    __syncthreads();
+    digit_start -= block_count;
+    global_start -= hist_d;
+    for (int w = 0; w < wave; ++w) {
+        digit_start += sm.tmp[0][w];
+        global_start += sm.tmp[1][w];
+    }
     if ((uint32_t)tid < R) {
         sm.digit_start[tid] = digit_start;
         sm.out_base[tid] = global_start + part_off - digit_start;
